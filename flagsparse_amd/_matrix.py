@@ -128,9 +128,7 @@ class CsrHandle:
         device = dC.device
         dB = dB if dB is not None else torch.empty((self.n_cols, n_dense), dtype=data.dtype, device=device)
         dvalues = dvalues if dvalues is not None else torch.empty(self.nnz, dtype=data.dtype, device=device)
-        vec = 16 // elem
-        wide = all(t.data_ptr() % 16 == 0 and int(t.stride(0)) % vec == 0 for t in (dC, B, dB)) and n_dense % vec == 0
-        if n_dense > 64 * (vec if wide else 1):
+        if n_dense > 64 * (16 // elem):
             return None
         G = _plan.lanes_for_dense(n_dense, elem)
         cfg = _plan.spmm_config(G)

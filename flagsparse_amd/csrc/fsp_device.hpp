@@ -40,20 +40,14 @@ template <typename T, typename A> __device__ __forceinline__ T from_acc(A v) {
 }
 
 // ------------------------------------------------------------ vector loads
-// VEC consecutive elements of T loaded / stored as one aligned access of
-// VEC*sizeof(T) bytes (<= 16).
-template <typename T, int VEC> struct alignas(sizeof(T) * VEC) vec_t {
+// VEC consecutive elements of T loaded / stored as one access of
+// VEC*sizeof(T) bytes (<= 16), aligned to one element only: gfx950 runs with
+// unaligned global access on, so the compiler emits the same dwordx4 for any
+// element-aligned address and a row of any length or stride is read 16 bytes
+// per lane.
+template <typename T, int VEC> struct vec_t {
   T v[VEC];
 };
-
-template <typename T, int VEC>
-__device__ __forceinline__ vec_t<T, VEC> load_vec(const T* p) {
-  return *reinterpret_cast<const vec_t<T, VEC>*>(p);
-}
-template <typename T, int VEC>
-__device__ __forceinline__ void store_vec(T* p, const vec_t<T, VEC>& v) {
-  *reinterpret_cast<vec_t<T, VEC>*>(p) = v;
-}
 
 // ---------------------------------------------------------- cross-lane moves
 // DPP control codes (GCN/CDNA ISA): quad_perm selectors, row mirrors.

@@ -38,7 +38,9 @@ __device__ __forceinline__ A transposed_sum4(const A (&dot)[4], int gl, int G, i
   return f;
 }
 
-template <typename T, typename IT, typename PT, int VEC, int UNROLL, bool ONE_CHUNK, bool OFF32>
+// TAIL: VEC does not divide K.  Its own instantiation, so whole-vector rows
+// pay for no mask.
+template <typename T, typename IT, typename PT, int VEC, int UNROLL, bool ONE_CHUNK, bool OFF32, bool TAIL>
 __global__ __launch_bounds__(FSP_WG_THREADS) void sddmm_bins_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const T* __restrict__ X, int64_t ldx,
     const T* __restrict__ Y, int64_t ldy, const T* __restrict__ data_in, T* __restrict__ out, int64_t k,
@@ -64,7 +66,18 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void sddmm_bins_kernel(
   const int64_t rr_step = tr.step * per_block;
   const O kk0 = static_cast<O>(gl) * VEC;
   const bool k_ok = static_cast<int64_t>(kk0) < k;
-  const O kk_ld = k_ok ? kk0 : O(0);  // lanes past K read column 0 (masked)
+  // When VEC does not divide K the vector that would leave the row is moved
+  // back to end at K (the host picks VEC <= K); the columns it then shares
+  // with its neighbour are zeroed on both sides, so each counts once.
+  auto inside = [&](O kk) { return !TAIL || static_cast<int64_t>(kk) + VEC <= k ? kk : static_cast<O>(k - VEC); };
+  auto drop_shared = [&](V& v, int ov) {
+#pragma unroll
+    for (int i = 0; i < VEC - 1; ++i) {
+      if (i < ov) v.v[i] = T(0);
+    }
+  };
+  const O kk_ld = k_ok ? inside(kk0) : O(0);  // lanes past K read column 0 (masked)
+  const int ov0 = k_ok ? static_cast<int>(kk0 - kk_ld) : 0;
   const O ldx_o = static_cast<O>(ldx), ldy_o = static_cast<O>(ldy);
   const int64_t last_item = lb.count - 1;
   const bool use_transposed = UNROLL == 4 && G >= 4;
@@ -139,6 +152,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void sddmm_bins_kernel(
         item(rr_next, row_n, beg_n, end_n);
         xv_n = *addr<OFF32>::at(reinterpret_cast<const V*>(X), (row_n * ldx_o + kk_ld) * static_cast<O>(sizeof(T)));
       }
+      if constexpr (TAIL) drop_shared(xv, ov0);
       A xr[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) xr[v] = k_ok ? static_cast<A>(xv.v[v]) : A(0);
@@ -158,6 +172,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void sddmm_bins_kernel(
         A dot[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
+          if constexpr (TAIL) drop_shared(yv[u], ov0);
           dot[u] = A(0);
 #pragma unroll
           for (int v = 0; v < VEC; ++v) dot[u] += xr[v] * static_cast<A>(yv[u].v[v]);
@@ -189,15 +204,19 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void sddmm_bins_kernel(
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) dot[u] = A(0);
         for (O kk = kk0; static_cast<int64_t>(kk) < k; kk += kstep) {
-          const V xv = *addr<OFF32>::at(reinterpret_cast<const V*>(X), (row * ldx_o + kk) * static_cast<O>(sizeof(T)));
+          const O kc = inside(kk);
+          const int ov = static_cast<int>(kk - kc);
+          V xv = *addr<OFF32>::at(reinterpret_cast<const V*>(X), (row * ldx_o + kc) * static_cast<O>(sizeof(T)));
           V yv[UNROLL];
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) {
             yv[u] = *addr<OFF32>::at(reinterpret_cast<const V*>(Y),
-                                     (static_cast<O>(c[u]) * ldy_o + kk) * static_cast<O>(sizeof(T)));
+                                     (static_cast<O>(c[u]) * ldy_o + kc) * static_cast<O>(sizeof(T)));
           }
+          if constexpr (TAIL) drop_shared(xv, ov);
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) {
+            if constexpr (TAIL) drop_shared(yv[u], ov);
 #pragma unroll
             for (int v = 0; v < VEC; ++v) dot[u] += static_cast<A>(xv.v[v]) * static_cast<A>(yv[u].v[v]);
           }
@@ -234,25 +253,34 @@ static int launch_sddmm(const void* indptr, const void* indices, const void* X, 
                      nnz * (int64_t)sizeof(IT) < lim && n_rows * ldx * (int64_t)sizeof(T) < lim &&
                      y_rows * ldy * (int64_t)sizeof(T) < lim;
   const dim3 grid(static_cast<unsigned>(blocks)), block(FSP_WG_THREADS);
-#define FSP_SDDMM_LAUNCH(ONE, O32)                                                                         \
-  hipLaunchKernelGGL((sddmm_bins_kernel<T, IT, PT, VEC, 4, ONE, O32>), grid, block, 0, s,                    \
+#define FSP_SDDMM_LAUNCH(ONE, O32, TAIL)                                                                    \
+  hipLaunchKernelGGL((sddmm_bins_kernel<T, IT, PT, VEC, 4, ONE, O32, TAIL>), grid, block, 0, s,              \
                      static_cast<const PT*>(indptr), static_cast<const IT*>(indices),                       \
                      static_cast<const T*>(X), ldx, static_cast<const T*>(Y), ldy,                          \
                      static_cast<const T*>(data_in), static_cast<T*>(out), k, static_cast<A>(alpha),        \
                      static_cast<A>(beta), g_log2, tab)
-  if (one_chunk) {
-    if (off32) {
-      FSP_SDDMM_LAUNCH(true, true);
-    } else {
-      FSP_SDDMM_LAUNCH(true, false);
-    }
-  } else {
-    if (off32) {
-      FSP_SDDMM_LAUNCH(false, true);
-    } else {
-      FSP_SDDMM_LAUNCH(false, false);
+#define FSP_SDDMM_WIDTH(TAIL)            \
+  if (one_chunk) {                       \
+    if (off32) {                         \
+      FSP_SDDMM_LAUNCH(true, true, TAIL);  \
+    } else {                             \
+      FSP_SDDMM_LAUNCH(true, false, TAIL); \
+    }                                    \
+  } else {                               \
+    if (off32) {                         \
+      FSP_SDDMM_LAUNCH(false, true, TAIL); \
+    } else {                             \
+      FSP_SDDMM_LAUNCH(false, false, TAIL); \
+    }                                    \
+  }
+  if constexpr (VEC > 1) {
+    if (k % VEC != 0) {
+      FSP_SDDMM_WIDTH(true);
+      return check_launch("sddmm_bins");
     }
   }
+  FSP_SDDMM_WIDTH(false);
+#undef FSP_SDDMM_WIDTH
 #undef FSP_SDDMM_LAUNCH
   return check_launch("sddmm_bins");
 }
@@ -282,10 +310,7 @@ extern "C" int fsp_sddmm_csr(int32_t value_type, int32_t index_type, int32_t ind
     FSP_DISPATCH_INDEX(index_type, IT, {
       FSP_DISPATCH_INDEX(indptr_type, PT, {
         constexpr int V = 16 / sizeof(T);
-        const bool wide = (reinterpret_cast<uintptr_t>(X_dev) % 16 == 0) &&
-                          (reinterpret_cast<uintptr_t>(Y_dev) % 16 == 0) && k % V == 0 && ldx % V == 0 &&
-                          ldy % V == 0;
-        if (wide) {
+        if (k >= V) {  // 16 bytes per lane for any K, stride and alignment of the rows
           return launch_sddmm<T, IT, PT, V>(indptr_dev, indices_dev, X_dev, ldx, Y_dev, ldy, data_in_dev, out_dev,
                                             n_rows, k, nnz, y_rows, alpha, beta, lanes_k, plan, s);
         }
