@@ -249,7 +249,7 @@ static int launch_sddmm(const void* indptr, const void* indices, const void* X, 
   if (blocks == 0) return FSP_OK;
   const bool one_chunk = vk <= G;
   const int64_t lim = int64_t(1) << 32;
-  const bool off32 = std::is_same<PT, int32_t>::value && nnz * (int64_t)sizeof(T) < lim &&
+  const bool off32 = nnz * (int64_t)sizeof(T) < lim &&
                      nnz * (int64_t)sizeof(IT) < lim && n_rows * ldx * (int64_t)sizeof(T) < lim &&
                      y_rows * ldy * (int64_t)sizeof(T) < lim;
   const dim3 grid(static_cast<unsigned>(blocks)), block(FSP_WG_THREADS);

@@ -392,21 +392,22 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
   }
   if (blocks > 0) {
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(ytiles));
-    // 32-bit byte offsets when every array the kernel addresses fits in 4 GiB.
+    // 32-bit byte offsets when every array the kernel addresses fits in 4 GiB,
+    // whatever the row pointer's type (its values fit then too).  With 64-bit
+    // pointers and 64-bit offsets the f64 N = 75 product above took 301 us
+    // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.
     const int64_t lim = int64_t(1) << 32;
-    const bool off32 = std::is_same<PT, int32_t>::value &&
-                       (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
+    const bool off32 = (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
                        x.nnz * (int64_t)sizeof(T) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
                        x.nnz * (int64_t)sizeof(QT) < lim && x.b_rows * x.ldb * (int64_t)sizeof(T) < lim &&
                        x.n_rows * x.ldc * (int64_t)sizeof(T) < lim && partial_bytes < lim &&
                        (!SDD || x.n_rows * x.ldbj * (int64_t)sizeof(T) < lim);
     if (off32) {
-      using P32 = int32_t;
       using Q32 = int32_t;
       if (plan->unroll >= 8) {
-        launch_bins<T, IT, P32, Q32, VEC, 8, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
+        launch_bins<T, IT, PT, Q32, VEC, 8, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
       } else {
-        launch_bins<T, IT, P32, Q32, VEC, 4, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
+        launch_bins<T, IT, PT, Q32, VEC, 4, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
       }
     } else {
       launch_bins<T, IT, PT, QT, VEC, 4, PERM, false, SDD>(x, grid, g_log2, partials, tab, s);
