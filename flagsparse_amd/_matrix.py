@@ -17,6 +17,10 @@ from . import _lib, _plan
 from ._csc import csr_to_csc_perm, gather_values
 
 
+# values wider than the dense operands: dense dtype -> value (and sum) dtype
+_WIDE_VALUES = {torch.float32: torch.float64, torch.bfloat16: torch.float32, torch.float16: torch.float32}
+
+
 def _acc_dtype(dtype):
     return torch.float64 if dtype == torch.float64 else torch.float32
 
@@ -67,17 +71,20 @@ class CsrHandle:
         kernel that loads data[perm[q]] itself puts that random read in every
         nonzero's dependent chain and measures 10-19 % slower (262144^2 power
         law at N = 64 and the 200000-node graph at N = 128, f32 and bf16).
-        values_via_perm=True keeps that form; both are bitwise equal."""
+        values_via_perm=True keeps that form; both are bitwise equal.
+        data may be wider than B (float64 values over float32 operands,
+        float32 over 16-bit ones): the sums are kept in data's dtype and C, in
+        B's dtype, is rounded once."""
         n_out = self.n_cols if transpose else self.n_rows
         n_dense = int(B.shape[1])
         device = B.device
-        C = out if out is not None else torch.empty((n_out, n_dense), dtype=data.dtype, device=device)
+        C = out if out is not None else torch.empty((n_out, n_dense), dtype=B.dtype, device=device)
         if n_out == 0 or n_dense == 0:
             return C
         if (self.n_rows if transpose else self.n_cols) == 0 or self.nnz == 0:
             C.zero_()
             return C
-        G = int(lanes_n) if lanes_n else _plan.lanes_for_dense(n_dense, data.element_size())
+        G = int(lanes_n) if lanes_n else _plan.lanes_for_dense(n_dense, B.element_size())
         cfg = config or _plan.spmm_config(G)
         if transpose:
             colptr, rowind, perm = self.csc()
@@ -90,6 +97,18 @@ class CsrHandle:
             ptr_t, idx_t, perm_t = self.indptr, self.indices, None
         partials = plan.partials(n_dense, _acc_dtype(data.dtype), device)
         st = plan.struct(partials, max_blocks, xcd_groups)
+        if data.dtype != B.dtype:
+            if perm_t is not None or _WIDE_VALUES.get(B.dtype) != data.dtype:
+                raise TypeError(f"no kernel for {data.dtype} values with {B.dtype} dense operands")
+            _lib.check(
+                _lib.load().fsp_spmm_csr_wide(
+                    _lib.value_code(B.dtype), _lib.index_code(idx_t.dtype), _lib.index_code(ptr_t.dtype),
+                    _lib.ptr(ptr_t), _lib.ptr(idx_t), _lib.ptr(data), B.data_ptr(), int(B.stride(0)), C.data_ptr(),
+                    int(C.stride(0)), n_out, n_dense, self.nnz, int(B.shape[0]), G, st, _lib.stream_ptr(device),
+                ),
+                "fsp_spmm_csr_wide",
+            )
+            return C
         _lib.check(
             _lib.load().fsp_spmm_csr(
                 _lib.value_code(data.dtype),

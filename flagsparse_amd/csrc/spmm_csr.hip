@@ -9,6 +9,9 @@ FSP_SPMM_INSTANCES(extern, float)
 FSP_SPMM_INSTANCES(extern, double)
 FSP_SPMM_INSTANCES(extern, __bf16)
 FSP_SPMM_INSTANCES(extern, _Float16)
+FSP_SPMM_WIDE_INSTANCE(extern, float, double)
+FSP_SPMM_WIDE_INSTANCE(extern, __bf16, float)
+FSP_SPMM_WIDE_INSTANCE(extern, _Float16, float)
 }  // namespace fsp
 
 // Scratch of the no-allocation SpMM entry: the long-row partials live in
@@ -56,7 +59,9 @@ static int current_scratch(void* stream, void** out) {
 static int spmm_entry(int32_t value_type, int32_t index_type, int32_t indptr_type, const void* indptr_dev,
                       const void* indices_dev, const void* data_dev, int32_t perm_type, const void* perm_dev,
                       const void* B_dev, int64_t ldb, void* C_dev, int64_t ldc, int64_t n_rows, int64_t n_dense,
-                      int64_t nnz, int64_t b_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream) {  if (n_rows < 0 || n_dense < 0 || nnz < 0 || b_rows < 0) return fail(FSP_ERR_ARG, "fsp_spmm_csr: negative size");
+                      int64_t nnz, int64_t b_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream,
+                      bool wide_values = false) {
+  if (n_rows < 0 || n_dense < 0 || nnz < 0 || b_rows < 0) return fail(FSP_ERR_ARG, "fsp_spmm_csr: negative size");
   int st = check_plan(plan, n_rows);
   if (st) return st;
   if (n_rows == 0 || n_dense == 0) return FSP_OK;
@@ -80,6 +85,13 @@ static int spmm_entry(int32_t value_type, int32_t index_type, int32_t indptr_typ
   if (indices_dev == nullptr || data_dev == nullptr || b_rows == 0) {
     return fail(FSP_ERR_ARG, "fsp_spmm_csr: NULL indices/data or empty B with nonzeros");
   }
+  if (wide_values) {
+    switch (value_type) {
+      case FSP_F32: return spmm_wide_launch<float, double>(index_type, indptr_type, x, plan, s);
+      case FSP_BF16: return spmm_wide_launch<__bf16, float>(index_type, indptr_type, x, plan, s);
+      default: return spmm_wide_launch<_Float16, float>(index_type, indptr_type, x, plan, s);
+    }
+  }
   FSP_DISPATCH_VALUE(value_type, T, { return spmm_launch<T>(index_type, indptr_type, perm_type, x, plan, s); });
   return FSP_OK;
 }
@@ -95,6 +107,17 @@ extern "C" int fsp_spmm_csr(int32_t value_type, int32_t index_type, int32_t indp
                             const fsp_csr_plan* plan, void* stream) {
   return spmm_entry(value_type, index_type, indptr_type, indptr_dev, indices_dev, data_dev, perm_type, perm_dev,
                     B_dev, ldb, C_dev, ldc, n_rows, n_dense, nnz, b_rows, lanes_n, plan, stream);
+}
+
+extern "C" int fsp_spmm_csr_wide(int32_t dense_type, int32_t index_type, int32_t indptr_type, const void* indptr_dev,
+                                 const void* indices_dev, const void* data_dev, const void* B_dev, int64_t ldb,
+                                 void* C_dev, int64_t ldc, int64_t n_rows, int64_t n_dense, int64_t nnz,
+                                 int64_t b_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream) {
+  if (dense_type != FSP_F32 && dense_type != FSP_BF16 && dense_type != FSP_F16) {
+    return fail(FSP_ERR_DTYPE, "fsp_spmm_csr_wide: dense type %d has no wider value type", (int)dense_type);
+  }
+  return spmm_entry(dense_type, index_type, indptr_type, indptr_dev, indices_dev, data_dev, 0, nullptr, B_dev, ldb,
+                    C_dev, ldc, n_rows, n_dense, nnz, b_rows, lanes_n, plan, stream, true);
 }
 
 extern "C" int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, int32_t indptr_type,

@@ -78,14 +78,19 @@ struct sdd_args {
 // TAIL (SDD only): VEC does not divide n_dense, see `ov`.  Its own
 // instantiation: as a branch on a uniform flag the masks cost the whole-vector
 // backward 9 % (bf16, N = 128).
-template <typename T, typename IT, typename PT, typename QT, int VEC, int UNROLL, bool PERM, bool OFF32, bool SDD,
+// TV: type of A's values, T itself or the wider type the COO product computes
+// in (f64 over f32, f32 over f16 / bf16).  Sums are kept in TV's accumulation
+// type either way; B and C stay in T, so what is gathered and written is half
+// the bytes of a product over widened copies of B and C, and the copies'
+// passes are gone: f32, 150001 x 90001, 3 M nonzeros, N = 100: 457 -> 207 us.
+template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, bool PERM, bool OFF32, bool SDD,
           bool TAIL>
 __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
-    const PT* __restrict__ indptr, const IT* __restrict__ indices, const T* __restrict__ data,
+    const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
     const QT* __restrict__ perm, const T* __restrict__ B, int64_t ldb, T* __restrict__ C, int64_t ldc,
-    int64_t n_dense, int g_log2, typename acc_of<T>::type* __restrict__ partials, launch_table tab,
+    int64_t n_dense, int g_log2, typename acc_of<TV>::type* __restrict__ partials, launch_table tab,
     sdd_args<T, QT> sd) {
-  using A = typename acc_of<T>::type;
+  using A = typename acc_of<TV>::type;
   using O = typename addr<OFF32>::off_t;  // element / byte offsets
   using P = typename std::conditional<OFF32, int32_t, int64_t>::type;  // nonzero positions
   const int k = find_bin(tab, blockIdx.x);
@@ -152,7 +157,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
   // stay raw: masking or converting them here would make the compiler wait
   // for every load in flight (the B rows included) right after the prefetch,
   // so the mask and the conversion are applied where they are consumed.
-  auto trip = [&](P p, P end, IT (&c)[UNROLL], T (&a)[UNROLL], QT (&pq)[UNROLL]) {
+  auto trip = [&](P p, P end, IT (&c)[UNROLL], TV (&a)[UNROLL], QT (&pq)[UNROLL]) {
     const P last = end > 0 ? end - 1 : P(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
@@ -179,7 +184,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
   P beg, end;
   item(rr, out, beg, end, jrow);
   IT c[UNROLL];
-  T a[UNROLL];
+  TV a[UNROLL];
   QT pq[UNROLL];
   trip(beg + slot, end, c, a, pq);
 
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
       const P pn = p + static_cast<P>(S) * UNROLL;
       const bool same = pn < end;
       prefetched = prefetched || !same;
-      T an[UNROLL];
+      TV an[UNROLL];
       IT cn[UNROLL];
       QT pqn[UNROLL];
       if constexpr (SDD) {
@@ -290,11 +295,10 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
 // range and output row are wave-uniform loads, lane l takes columns l,
 // l + 64, ..., and each segment's partial row is one coalesced read whose
 // address does not depend on the previous one.
-template <typename T>
+template <typename T, typename A>
 __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_long_reduce_kernel(
-    const typename acc_of<T>::type* __restrict__ partials, const int32_t* __restrict__ long_rows,
+    const A* __restrict__ partials, const int32_t* __restrict__ long_rows,
     const int64_t* __restrict__ seg_ptr, int64_t n_long, int64_t n_dense, T* __restrict__ C, int64_t ldc) {
-  using A = typename acc_of<T>::type;
   const int lane = threadIdx.x & 63;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * FSP_WAVES + (threadIdx.x >> 6); i < n_long;
        i += static_cast<int64_t>(gridDim.x) * FSP_WAVES) {
@@ -343,29 +347,30 @@ struct spmm_args {
   void* dvals = nullptr;
 };
 
-template <typename T, typename IT, typename PT, typename QT, int VEC, int UNROLL, bool PERM, bool OFF32, bool SDD>
-static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_of<T>::type* partials,
+template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, bool PERM, bool OFF32,
+          bool SDD>
+static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_of<TV>::type* partials,
                         const launch_table& tab, hipStream_t s) {
   const sdd_args<T, QT> sd{static_cast<const T*>(x.Bj), x.ldbj, static_cast<const QT*>(x.pos),
                            static_cast<T*>(x.dvals)};
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(FSP_WG_THREADS), 0, s, static_cast<const PT*>(x.indptr),
-                       static_cast<const IT*>(x.indices), static_cast<const T*>(x.data),
+                       static_cast<const IT*>(x.indices), static_cast<const TV*>(x.data),
                        static_cast<const QT*>(x.perm), static_cast<const T*>(x.B), x.ldb, static_cast<T*>(x.C),
                        x.ldc, x.n_dense, g_log2, partials, tab, sd);
   };
   if constexpr (SDD && VEC > 1) {
     if (x.n_dense % VEC != 0) {
-      launch(spmm_bins_kernel<T, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, true>);
+      launch(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, true>);
       return;
     }
   }
-  launch(spmm_bins_kernel<T, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, false>);
+  launch(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, false>);
 }
 
-template <typename T, typename IT, typename PT, typename QT, int VEC, bool PERM, bool SDD>
+template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, bool PERM, bool SDD>
 static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t s) {
-  using A = typename acc_of<T>::type;
+  using A = typename acc_of<TV>::type;
   const int64_t vcols = ceil_div(x.n_dense, VEC);
   int G = x.lanes_n;
   if (G <= 0) {
@@ -398,19 +403,19 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
     // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.
     const int64_t lim = int64_t(1) << 32;
     const bool off32 = (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
-                       x.nnz * (int64_t)sizeof(T) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
+                       x.nnz * (int64_t)sizeof(TV) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
                        x.nnz * (int64_t)sizeof(QT) < lim && x.b_rows * x.ldb * (int64_t)sizeof(T) < lim &&
                        x.n_rows * x.ldc * (int64_t)sizeof(T) < lim && partial_bytes < lim &&
                        (!SDD || x.n_rows * x.ldbj * (int64_t)sizeof(T) < lim);
     if (off32) {
       using Q32 = int32_t;
       if (plan->unroll >= 8) {
-        launch_bins<T, IT, PT, Q32, VEC, 8, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
+        launch_bins<T, TV, IT, PT, Q32, VEC, 8, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
       } else {
-        launch_bins<T, IT, PT, Q32, VEC, 4, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
+        launch_bins<T, TV, IT, PT, Q32, VEC, 4, PERM, true, SDD>(x, grid, g_log2, partials, tab, s);
       }
     } else {
-      launch_bins<T, IT, PT, QT, VEC, 4, PERM, false, SDD>(x, grid, g_log2, partials, tab, s);
+      launch_bins<T, TV, IT, PT, QT, VEC, 4, PERM, false, SDD>(x, grid, g_log2, partials, tab, s);
     }
     const int st = check_launch("spmm_bins");
     if (st) return st;
@@ -418,7 +423,7 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
   if (plan->n_long_rows > 0) {
     int64_t g = ceil_div(plan->n_long_rows, FSP_WAVES);
     if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(spmm_long_reduce_kernel<T>, dim3(static_cast<unsigned>(g)), dim3(FSP_WG_THREADS), 0, s,
+    hipLaunchKernelGGL((spmm_long_reduce_kernel<T, A>), dim3(static_cast<unsigned>(g)), dim3(FSP_WG_THREADS), 0, s,
                        partials, plan->long_rows_dev, plan->long_seg_ptr_dev, plan->n_long_rows, x.n_dense,
                        static_cast<T*>(x.C), x.ldc);
     return check_launch("spmm_long_reduce");
@@ -426,16 +431,16 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
   return FSP_OK;
 }
 
-template <typename T, typename IT, typename PT, typename QT, bool PERM, bool SDD = false>
+template <typename T, typename TV, typename IT, typename PT, typename QT, bool PERM, bool SDD = false>
 static int launch_spmm_vec(spmm_args x, const fsp_csr_plan* plan, hipStream_t s) {
   // 16 bytes per lane whatever the width, stride and alignment of the dense
   // rows, as long as a row holds one vector.  The element-wise form (VEC 1)
   // needs a lane per column: 75 f64 columns took two 64-lane column tiles of
   // 8-byte loads, 503 us against 301 us here (100003 x 70001, 2.4 M nonzeros).
   constexpr int V = 16 / sizeof(T);
-  if (x.n_dense >= V) return launch_spmm<T, IT, PT, QT, V, PERM, SDD>(x, plan, s);
+  if (x.n_dense >= V) return launch_spmm<T, TV, IT, PT, QT, V, PERM, SDD>(x, plan, s);
   x.lanes_n = 0;
-  return launch_spmm<T, IT, PT, QT, 1, PERM, SDD>(x, plan, s);
+  return launch_spmm<T, TV, IT, PT, QT, 1, PERM, SDD>(x, plan, s);
 }
 
 // Kernel launches of one value type over the index types.  Each value type is
@@ -446,8 +451,8 @@ int spmm_launch(int32_t index_type, int32_t indptr_type, int32_t perm_type, cons
                 const fsp_csr_plan* plan, hipStream_t s) {
   FSP_DISPATCH_INDEX(index_type, IT, {
     FSP_DISPATCH_INDEX(indptr_type, PT, {
-      if (x.perm == nullptr) return launch_spmm_vec<T, IT, PT, int32_t, false>(x, plan, s);
-      FSP_DISPATCH_INDEX(perm_type, QT, { return launch_spmm_vec<T, IT, PT, QT, true>(x, plan, s); });
+      if (x.perm == nullptr) return launch_spmm_vec<T, T, IT, PT, int32_t, false>(x, plan, s);
+      FSP_DISPATCH_INDEX(perm_type, QT, { return launch_spmm_vec<T, T, IT, PT, QT, true>(x, plan, s); });
     });
   });
   return FSP_OK;
@@ -458,11 +463,24 @@ int spmm_sdd_launch(int32_t index_type, int32_t indptr_type, int32_t pos_type, c
                     const fsp_csr_plan* plan, hipStream_t s) {
   FSP_DISPATCH_INDEX(index_type, IT, {
     FSP_DISPATCH_INDEX(indptr_type, PT, {
-      FSP_DISPATCH_INDEX(pos_type, QT, { return launch_spmm_vec<T, IT, PT, QT, false, true>(x, plan, s); });
+      FSP_DISPATCH_INDEX(pos_type, QT, { return launch_spmm_vec<T, T, IT, PT, QT, false, true>(x, plan, s); });
     });
   });
   return FSP_OK;
 }
+
+// Values in the wider type TV (see spmm_bins_kernel).
+template <typename T, typename TV>
+int spmm_wide_launch(int32_t index_type, int32_t indptr_type, const spmm_args& x, const fsp_csr_plan* plan,
+                     hipStream_t s) {
+  FSP_DISPATCH_INDEX(index_type, IT, {
+    FSP_DISPATCH_INDEX(indptr_type, PT, { return launch_spmm_vec<T, TV, IT, PT, int32_t, false>(x, plan, s); });
+  });
+  return FSP_OK;
+}
+
+#define FSP_SPMM_WIDE_INSTANCE(EXTERN, T, TV) \
+  EXTERN template int spmm_wide_launch<T, TV>(int32_t, int32_t, const spmm_args&, const fsp_csr_plan*, hipStream_t);
 
 #define FSP_SPMM_INSTANCES(EXTERN, T)                                                                          \
   EXTERN template int spmm_launch<T>(int32_t, int32_t, int32_t, const spmm_args&, const fsp_csr_plan*, hipStream_t); \

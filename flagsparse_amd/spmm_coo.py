@@ -8,8 +8,10 @@ float16 / bfloat16 in float32, and the result is cast to the input dtype.
 
 Here the canonical order comes from the stable HIP COO -> CSR conversion
 (``fsp_coo_to_csr``, values moved bit-exactly) and every route runs the HIP
-row-bin SpMM (``fsp_spmm_csr``) over that CSR in the same compute dtype, so
-no atomics are involved and results are deterministic.  Duplicate (row, col)
+row-bin SpMM over that CSR: the values are held in the compute dtype, B and C
+stay in the input dtype, and the kernel (``fsp_spmm_csr_wide``) widens B's
+elements as it multiplies, sums in the compute dtype and rounds C once.  No
+atomics are involved and results are deterministic.  Duplicate (row, col)
 entries stay as separate nonzeros in (row, col) order and the kernel sums
 them (the reference sums them first; the two agree up to rounding).  Names,
 arguments, validation order, messages, returns, meta keys and the dense
@@ -166,19 +168,23 @@ class _CanonicalCoo:
         self.shape = (n_rows, n_cols)
         self.handle = CsrHandle(indices, indptr, self.shape)
 
-    def spmm(self, B_compute, output_dtype, dense_layout, out=None):
-        """C = op(A) B in the requested layout and dtype (row-major kernel)."""
+    def spmm(self, B, dense_layout, out=None):
+        """C = op(A) B in the requested layout (row-major kernel): B and C in
+        the input dtype, products and sums in the values' compute dtype."""
         n_rows = self.shape[0]
-        n_dense = int(B_compute.shape[1])
-        C_acc = self.handle.spmm(self.data, B_compute.contiguous())
+        B_row = B.contiguous()
+        # the kernel writes a contiguous `out` itself unless it is B's own
+        # memory; an `out` in the autograd graph gets copy_'s checks
+        direct = (out if out is not None and out.is_contiguous() and not out.requires_grad
+                  and out.untyped_storage().data_ptr() != B_row.untyped_storage().data_ptr() else None)
+        C_row = self.handle.spmm(self.data, B_row, out=direct)
         if out is not None:
-            out.copy_(C_acc)
-            return out
+            return out if direct is not None else out.copy_(C_row)
         if dense_layout == "col":
-            C = _empty_dense_layout((n_rows, n_dense), output_dtype, C_acc.device, "col")
-            C.copy_(C_acc)
+            C = _empty_dense_layout((n_rows, int(B.shape[1])), B.dtype, C_row.device, "col")
+            C.copy_(C_row)
             return C
-        return C_acc if C_acc.dtype == output_dtype else C_acc.to(output_dtype)
+        return C_row
 
 
 @dataclass(frozen=True)
@@ -239,22 +245,25 @@ def _validate_spmm_coo_route_runtime_inputs(prepared, B, dense_layout):
         raise TypeError("B dtype must match sparse matrix dtype")
     if int(B.shape[0]) != prepared.n_cols:
         raise ValueError(f"B.shape[0] must be n_cols={prepared.n_cols}, got {B.shape[0]}")
-    B_compute = B if prepared.compute_dtype == prepared.output_dtype else B.to(prepared.compute_dtype)
-    return _materialize_dense_layout(B_compute, dense_layout)
+    if dense_layout == "col" and prepared.compute_dtype != prepared.output_dtype:
+        span = 1 + sum((int(n) - 1) * abs(int(st)) for n, st in zip(B.shape, B.stride()))
+        if span != B.numel():  # a padded B keeps its order but not its gaps, as a widened copy does
+            B = B.clone()
+    return _materialize_dense_layout(B, dense_layout)
 
 
 def _route_runner(name, display_name):
     def run(prepared, B, *, timing=False, diagnostics=False, dense_layout="row"):
         dense_layout = _normalize_dense_layout(dense_layout)
         t_cpu = time.perf_counter()
-        B_compute = _validate_spmm_coo_route_runtime_inputs(prepared, B, dense_layout)
+        B = _validate_spmm_coo_route_runtime_inputs(prepared, B, dense_layout)
         process_cpu_ms = (time.perf_counter() - t_cpu) * 1000.0
         compute_ms = None
         if timing:
             start = torch.cuda.Event(enable_timing=True)
             end = torch.cuda.Event(enable_timing=True)
             start.record()
-        C = prepared._canonical.spmm(B_compute, prepared.output_dtype, dense_layout)
+        C = prepared._canonical.spmm(B, dense_layout)
         if timing:
             end.record()
             torch.cuda.synchronize()
@@ -266,7 +275,7 @@ def _route_runner(name, display_name):
             "process_gpu_ms": 0.0 if timing else None,
             "compute_ms": compute_ms,
             "dense_layout": dense_layout,
-            "b_stride": tuple(int(v) for v in B_compute.stride()),
+            "b_stride": tuple(int(v) for v in B.stride()),
             "c_stride": tuple(int(v) for v in C.stride()),
             "output_layout": _dense_layout_name(C),
         }
@@ -429,11 +438,10 @@ def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, o
             raise ValueError("out must be on the same CUDA device as the inputs")
         if tuple(out.shape) != (n_rows, n_dense) or out.dtype != output_dtype:
             raise ValueError("out shape/dtype must match result")
-    B_compute = B if compute_dtype == output_dtype else B.to(compute_dtype)
     if do_timing:
         torch.cuda.synchronize()
         t1 = time.perf_counter()
-    C = canonical.spmm(B_compute, output_dtype, dense_layout, out=out)
+    C = canonical.spmm(B, dense_layout, out=out)
     compute_ms = op_total_ms = None
     if do_timing:
         torch.cuda.synchronize()
@@ -448,7 +456,7 @@ def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, o
             "compute_ms": compute_ms,
             "op_total_ms": op_total_ms,
             "dense_layout": dense_layout,
-            "b_stride": tuple(int(v) for v in B_compute.stride()),
+            "b_stride": tuple(int(v) for v in B.stride()),
             "c_stride": tuple(int(v) for v in C.stride()),
             "output_layout": _dense_layout_name(C),
         }

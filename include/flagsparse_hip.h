@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FSP_ABI_VERSION 15
+#define FSP_ABI_VERSION 16
 #define FSP_MAX_BINS 8
 
 typedef enum fsp_value_type {
@@ -207,6 +207,19 @@ int fsp_spmm_csr(int32_t value_type, int32_t index_type, int32_t indptr_type,
                  int64_t n_rows, int64_t n_dense, int64_t nnz, int64_t b_rows,
                  int32_t lanes_n, const fsp_csr_plan* plan, void* stream);
 
+/* fsp_spmm_csr without a permutation whose values are wider than the dense
+ * operands: `dense_type` FSP_F32 takes f64 values and sums in f64, FSP_BF16 /
+ * FSP_F16 take f32 values and sum in f32; B and C are dense_type, C rounded
+ * once.  The numerics of the COO SpMM (spmm_coo.py:146-153), whose reference
+ * widens B and the result instead.  The plan's partials hold f64 (dense_type
+ * FSP_F32) or f32 sums; other dense types return FSP_ERR_DTYPE. */
+int fsp_spmm_csr_wide(int32_t dense_type, int32_t index_type, int32_t indptr_type,
+                      const void* indptr_dev, const void* indices_dev,
+                      const void* data_dev, const void* B_dev, int64_t ldb,
+                      void* C_dev, int64_t ldc, int64_t n_rows, int64_t n_dense,
+                      int64_t nnz, int64_t b_rows, int32_t lanes_n,
+                      const fsp_csr_plan* plan, void* stream);
+
 /* The differentiable SpMM's backward in one pass over A's CSC.  No
  * counterpart in the reference, which has no autograd; it computes what the
  * reference's trans SpMM (spmm_csr.py:3981, op trans) and
@@ -220,11 +233,10 @@ int fsp_spmm_csr(int32_t value_type, int32_t index_type, int32_t indptr_type,
  * n_cols x n_dense (ldb, lddb); dvalues has nnz entries in CSR order.
  * `plan` is the plan of the CSC (long columns as segments, partials as
  * fsp_spmm_csr).  dB is bitwise equal to fsp_spmm_csr over the same CSC and
- * plan (with B's rows 16-byte aligned wherever dC's and dB's are); dvalues
+ * plan; dvalues
  * are f32 (f64 for f64) dot products in the lanes' order.
  * n_dense must fit one lane group (64 lanes x 16 bytes: 256 f32 / 512
- * bf16 or f16 / 128 f64 columns on 16-byte aligned rows, else 64 columns);
- * wider operands return FSP_ERR_ARG and the caller runs the two kernels. */
+ * bf16 or f16 / 128 f64 columns); wider operands return FSP_ERR_ARG and the caller runs the two kernels. */
 int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, int32_t indptr_type,
                              const void* colptr_dev, const void* rowind_dev,
                              const void* data_csc_dev, int32_t pos_type, const void* pos_dev,
