@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 #define FSP_WG_THREADS 256
 #define FSP_WAVES (FSP_WG_THREADS / 64)
@@ -116,6 +117,36 @@ template <typename A> __device__ __forceinline__ A group_sum(A v, int lanes) {
   if (lanes >= 32) v += shfl_xor(v, 16);
   if (lanes >= 64) v += shfl_xor(v, 32);
   return v;
+}
+
+// Broadcast inside a lane group: every lane receives the value of lane U of
+// its quad (LANES 4) or of its row of 16 lanes (LANES 16).  One DPP move that
+// the compiler folds into an integer add where it can.
+template <int LANES, int U> __device__ __forceinline__ int bcast_i32(int v) {
+  static_assert((LANES == 4 || LANES == 16) && U >= 0 && U < LANES, "a quad or a row of 16 lanes");
+  constexpr int ctrl = LANES == 4 ? U * 0x55 : 0x150 + U;  // quad_perm [U,U,U,U] / row_newbcast:U
+  return __builtin_amdgcn_mov_dpp(v, ctrl, 0xF, 0xF, true);
+}
+template <int LANES, int U, typename V> __device__ __forceinline__ V bcast(V v) {
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, bcast_i32<LANES, U>(__builtin_bit_cast(int, v)));
+  } else {
+    static_assert(sizeof(V) == 8, "32- or 64-bit values");
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = static_cast<uint32_t>(bcast_i32<LANES, U>(static_cast<int>(static_cast<uint32_t>(u))));
+    const uint32_t hi = static_cast<uint32_t>(bcast_i32<LANES, U>(static_cast<int>(static_cast<uint32_t>(u >> 32))));
+    return __builtin_bit_cast(V, (static_cast<uint64_t>(hi) << 32) | lo);
+  }
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop
+// whose index is a constant expression (DPP controls are immediates).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // Byte-offset addressing: 32-bit offsets from a uniform base when OFF32.

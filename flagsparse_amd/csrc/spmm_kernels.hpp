@@ -85,7 +85,7 @@ struct sdd_args {
 // passes are gone: f32, 150001 x 90001, 3 M nonzeros, N = 100: 457 -> 207 us.
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, bool PERM, bool OFF32, bool SDD,
           bool TAIL>
-__global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
+__global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
     const QT* __restrict__ perm, const T* __restrict__ B, int64_t ldb, T* __restrict__ C, int64_t ldc,
     int64_t n_dense, int g_log2, typename acc_of<TV>::type* __restrict__ partials, launch_table tab,
@@ -290,6 +290,257 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_bins_kernel(
   }
 }
 
+// Third word of a raw buffer descriptor (32-bit elements, no swizzle).
+constexpr int kRawBuffer = 0x00020000;
+
+// n elements of E (below 4 GiB) as a buffer: element kAbsent reads as zero and
+// touches no memory.
+constexpr uint32_t kAbsent = ~0u;
+
+// B of at least twice the eight 4 MiB L2s, read in rows of 256 bytes or more:
+// nearly every gather crosses the fabric, and more of them in flight lowers its
+// throughput (262144^2, f32: N = 64 233 us with spmm_bins_kernel, 227 us with
+// five workgroups per CU, 228 us with spmm_slots_kernel; N = 160 558 against
+// 543 us).  Below that size the faster issue wins (200000-node graph, bf16
+// N = 128: 86 against 89 us; 50000 nodes, f32 N = 64: 24 against 26 us).
+constexpr int64_t kPacedBytes = int64_t(64) << 20;
+template <typename E>
+struct buffer {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ buffer(const E* p, uint32_t n)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<E*>(p), 0, n * static_cast<uint32_t>(sizeof(E)), kRawBuffer)) {}
+  __device__ __forceinline__ E load(uint32_t i) const {
+    const uint32_t off = i == kAbsent ? kAbsent : i * static_cast<uint32_t>(sizeof(E));
+    if constexpr (sizeof(E) == 2) {
+      return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0));
+    } else if constexpr (sizeof(E) == 4) {
+      return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
+    } else {
+      return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0));
+    }
+  }
+};
+
+// Workgroups per CU (waves per SIMD) the registers must allow.
+template <int UNROLL, bool SDD>
+constexpr int kMinBlocks = SDD ? 5 : (UNROLL > 4 ? 6 : 8);
+
+// The same layout and summation order as spmm_slots_kernel (bitwise equal),
+// with the id and value of a nonzero loaded once per quad (LANES 4) or row of
+// 16 lanes (LANES 16) instead of once per lane: lane q holds nonzero q of the
+// trip, computes its B row offset, and one DPP move per nonzero hands offset
+// and value to the group.  A wave load costs the CU's address unit 18 clocks
+// whatever its lanes ask for (measured: all lanes, half masked off, half out
+// of range), so two of every three loads, and the offset arithmetic of every
+// lane, are what goes.  Nonzeros past a row's end have their B row outside the
+// buffer: it reads as zeros without memory traffic, so nothing is masked and
+// no load is repeated, and the batches of UNROLL rows that no lane needs are
+// skipped.  Vector instructions per launch fell from 45.2 to 24.1 million and
+// loads from 6.1 to 2.6 million (262144^2, N = 64).  100003 x 70001 f64,
+// N = 75: 290 -> 242 us; 1024-matrix batch, N = 32: 686 -> 664 us;
+// 200000-node graph, bf16 N = 128: 89 -> 86 us, its backward 144 -> 141 us.
+template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool SDD,
+          bool TAIL>
+__global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spmm_bins_kernel(
+    const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
+    const T* __restrict__ B, int64_t ldb, uint32_t b_bytes, T* __restrict__ C, int64_t ldc, int64_t n_dense, uint32_t nnz,
+    int g_log2, typename acc_of<TV>::type* __restrict__ partials, launch_table tab, sdd_args<T, QT> sd) {
+  using A = typename acc_of<TV>::type;
+  constexpr bool OFF32 = true;
+  using O = uint32_t;  // element / byte offsets
+  using P = int32_t;   // nonzero positions
+  using V = vec_t<T, VEC>;
+  constexpr int kRegs = UNROLL > LANES ? UNROLL / LANES : 1;  // nonzeros a lane holds
+  constexpr int kTrip = LANES * kRegs;                         // nonzeros of a slot per trip
+  const launch_bin lb = tab.b[find_bin(tab, blockIdx.x)];  // a copy: the fields stay in registers
+  const int s_log2 = lb.lanes_log2;
+  const int G = 1 << g_log2;
+  const int S = 1 << s_log2;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int gl = lane & (G - 1);
+  const int slot = (lane >> g_log2) & (S - 1);
+  const int sub = lane >> (g_log2 + s_log2);
+  const int ql = lane & (LANES - 1);
+  const int64_t per_wave = 64 >> (g_log2 + s_log2);
+  const int64_t per_block = per_wave * FSP_WAVES;
+  // A lane's VEC columns, see spmm_slots_kernel.
+  const int64_t colv = (static_cast<int64_t>(blockIdx.y) * G + gl) * VEC;
+  const bool col_ok = colv < n_dense;
+  const O col0 = static_cast<O>(colv + VEC <= n_dense ? colv : n_dense - VEC);
+  const int ov = col_ok ? static_cast<int>(colv - static_cast<int64_t>(col0)) : 0;
+  const O col_off = (col_ok ? col0 : O(0)) * static_cast<O>(sizeof(T));  // lanes past n_dense read column 0
+  const tile_range tr = bin_tiles(lb, per_block);
+  const int64_t rr_step = tr.step * per_block;
+  const O row_bytes = static_cast<O>(ldb) * static_cast<O>(sizeof(T));
+  const int64_t last_item = lb.count - 1;  // bins in the table are non-empty
+  // B as a buffer of b_bytes: a load from `outside` (plus any column) reads
+  // zeros and touches no memory.
+  const auto brsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(B), 0, b_bytes, kRawBuffer);
+  const O outside = ~O(0) - row_bytes;
+  const buffer<IT> indices_b(indices, nnz);
+  const buffer<TV> data_b(data, nnz);
+  const buffer<QT> pos_b(sd.pos, nnz);
+
+  // Item (row or segment) of this lane; every lane of a group keeps the
+  // nonzero range, also past n_dense: the group's broadcasts read all of them.
+  auto item = [&](int64_t r, O& out, P& beg, P& end, O& jrow) {
+    const bool live = r < lb.count;
+    const int64_t rc = live ? r : last_item;
+    P b, e;
+    if (lb.is_segment) {
+      out = static_cast<O>(rc);
+      jrow = SDD ? static_cast<O>(tab.seg_row[rc]) : O(0);
+      b = static_cast<P>(tab.seg_begin[rc]);
+      e = static_cast<P>(tab.seg_end[rc]);
+    } else {
+      const int64_t row = lb.rows ? static_cast<int64_t>(lb.rows[rc]) : rc;
+      out = jrow = static_cast<O>(row);
+      b = static_cast<P>(indptr[row]);
+      e = static_cast<P>(indptr[row + 1]);
+    }
+    beg = live ? b : P(0);
+    end = live ? e : P(0);
+  };
+  // This lane's nonzeros of a trip that starts at the slot's nonzero p; past
+  // `end` they read as zero.
+  auto trip = [&](P p, P end, IT (&c)[kRegs], TV (&a)[kRegs], QT (&pq)[kRegs]) {
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) {
+      const P q = p + (static_cast<P>(r * LANES + ql) << s_log2);
+      const O at = q < end ? static_cast<O>(q) : kAbsent;
+      c[r] = indices_b.load(at);
+      a[r] = data_b.load(at);
+      if constexpr (SDD) pq[r] = pos_b.load(at);
+    }
+  };
+
+  int64_t rr = tr.first * per_block + wave * per_wave + sub;
+  O out, jrow;
+  P beg, end;
+  item(rr, out, beg, end, jrow);
+  IT c[kRegs];
+  TV a[kRegs];
+  QT pq[kRegs];
+  trip(beg + slot, end, c, a, pq);
+
+  for (int64_t tile = tr.first; tile < tr.end; tile += tr.step) {  // wave-uniform
+    const bool active = rr < lb.count && col_ok;
+    const int64_t rr_next = rr + rr_step;
+    // the next item is prefetched only when this workgroup will process it
+    const bool has_next = tile + tr.step < tr.end;  // wave-uniform
+    O out_n = 0, jrow_n = 0;
+    P beg_n = 0, end_n = 0;
+    if (has_next) item(rr_next, out_n, beg_n, end_n, jrow_n);
+    V bj;
+    if constexpr (SDD) {  // row j of the forward's B
+      bj = *addr<OFF32>::at(reinterpret_cast<const V*>(sd.Bj),
+                            jrow * static_cast<O>(sd.ldbj) * static_cast<O>(sizeof(T)) + col_off);
+      if constexpr (TAIL) {
+#pragma unroll
+        for (int v = 0; v < VEC - 1; ++v) bj.v[v] = v < ov ? T(0) : bj.v[v];
+      }
+    }
+    A acc[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) acc[v] = A(0);
+    P p = beg + slot;
+    bool prefetched = false;  // wave-uniform
+    while (__ballot(p < end) != 0) {  // wave-uniform: every lane takes part in the broadcasts
+      O off[kRegs];
+      A av[kRegs];
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) {
+        const bool ok = p + (static_cast<P>(r * LANES + ql) << s_log2) < end;
+        off[r] = ok ? static_cast<O>(c[r]) * row_bytes : outside;
+        av[r] = static_cast<A>(a[r]);
+      }
+      const P pn = p + (static_cast<P>(kTrip) << s_log2);
+      const bool same = pn < end;
+      IT cn[kRegs];
+      TV an[kRegs];
+      QT pqn[kRegs];
+      A dots[kRegs];
+      static_for<kTrip / UNROLL>([&](auto batch) {
+        constexpr int u0 = decltype(batch)::value * UNROLL;
+        if (u0 > 0 && __ballot(p + (static_cast<P>(u0) << s_log2) < end) == 0) return;  // wave-uniform
+        V b[UNROLL];
+        static_for<UNROLL>([&](auto u) {
+          constexpr int n = u0 + decltype(u)::value;
+          b[u] = __builtin_bit_cast(
+              V, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bcast<LANES, n % LANES>(off[n / LANES]) + col_off, 0, 0));
+        });
+        // prefetch: the next trip of this item, else the first trip of the
+        // next.  Unconditional (with nothing next it touches no memory): under
+        // a branch the compiler could not count the loads in flight, and the
+        // last B row of the batch would wait for the prefetch too.
+        if constexpr (u0 == 0) trip(same ? pn : beg_n + slot, same ? end : end_n, cn, an, pqn);
+        static_for<UNROLL>([&](auto u) {
+          constexpr int n = u0 + decltype(u)::value;
+          const A x = bcast<LANES, n % LANES>(av[n / LANES]);
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) acc[v] += x * static_cast<A>(b[u].v[v]);
+        });
+        if constexpr (SDD) {
+          // the dots of this batch: a lane's VEC products, then the sum over
+          // the slot's G lanes; the lane that holds the nonzero keeps it
+          static_for<UNROLL>([&](auto u) {
+            constexpr int n = u0 + decltype(u)::value;
+            V bu = b[u];
+            if constexpr (TAIL) {  // the shared columns count once, in the previous lane
+#pragma unroll
+              for (int v = 0; v < VEC - 1; ++v) bu.v[v] = v < ov ? T(0) : bu.v[v];
+            }
+            const A d = group_sum(col_ok ? row_dot<A>(bu, bj) : A(0), G);
+            dots[n / LANES] = ql == n % LANES ? d : dots[n / LANES];
+          });
+        }
+      });
+      if constexpr (SDD) {
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) {
+          const bool ok = p + (static_cast<P>(r * LANES + ql) << s_log2) < end;
+          if (ok && gl < LANES) {
+            *addr<OFF32>::at(sd.dvals, static_cast<O>(pq[r]) * static_cast<O>(sizeof(T))) = static_cast<T>(dots[r]);
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) {
+        c[r] = cn[r];
+        a[r] = an[r];
+        if constexpr (SDD) pq[r] = pqn[r];
+      }
+      p = pn;
+      prefetched = true;
+    }
+    if (!prefetched && has_next) trip(beg_n + slot, end_n, c, a, pq);
+    // Sum the S slots of a row: lanes that differ only in the slot bits.
+    for (int j = 0; j < s_log2; ++j) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) acc[v] += shfl_xor(acc[v], G << j);
+    }
+    if (active && slot == 0) {
+      if (lb.is_segment) {
+        A* dst = addr<OFF32>::at(partials, (out * static_cast<O>(n_dense) + col0) * static_cast<O>(sizeof(A)));
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) dst[v] = acc[v];
+      } else {
+        V o;
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) o.v[v] = static_cast<T>(acc[v]);
+        *addr<OFF32>::at(reinterpret_cast<V*>(C),
+                         (out * static_cast<O>(ldc) + col0) * static_cast<O>(sizeof(T))) = o;
+      }
+    }
+    out = out_n;
+    jrow = jrow_n;
+    beg = beg_n;
+    end = end_n;
+    rr = rr_next;
+  }
+}
+
 // C[long_rows[i], :] = sum of the row's segment partials, in segment order.
 // One wave per long row (a grid-stride loop over rows): the row's segment
 // range and output row are wave-uniform loads, lane l takes columns l,
@@ -353,6 +604,38 @@ static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_
                         const launch_table& tab, hipStream_t s) {
   const sdd_args<T, QT> sd{static_cast<const T*>(x.Bj), x.ldbj, static_cast<const QT*>(x.pos),
                            static_cast<T*>(x.dvals)};
+  // Groups of 4 or more lanes of whole vectors share their nonzeros through
+  // broadcasts; narrower groups, and values read through a permutation, load
+  // them per lane.
+  const int64_t b_bytes = x.b_rows * x.ldb * (int64_t)sizeof(T);
+  if constexpr (VEC > 1 && !PERM && OFF32) {
+    const auto bins = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(FSP_WG_THREADS), 0, s, static_cast<const PT*>(x.indptr),
+                         static_cast<const IT*>(x.indices), static_cast<const TV*>(x.data),
+                         static_cast<const T*>(x.B), x.ldb, static_cast<uint32_t>(b_bytes), static_cast<T*>(x.C), x.ldc,
+                         x.n_dense, static_cast<uint32_t>(x.nnz), g_log2, partials, tab, sd);
+    };
+    const auto width = [&](auto tail) {
+      constexpr bool TAIL = decltype(tail)::value;
+      if (g_log2 >= 4) {
+        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 16, SDD, TAIL>);
+      } else {
+        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 4, SDD, TAIL>);
+      }
+    };
+    // (b_bytes + a row stays below the offset that marks an absent nonzero)
+    const bool paced = g_log2 >= 4 && !SDD && b_bytes >= kPacedBytes;
+    if (g_log2 >= 2 && !paced && b_bytes <= (int64_t(1) << 32) - 1 - x.ldb * (int64_t)sizeof(T)) {
+      if constexpr (SDD) {
+        if (x.n_dense % VEC != 0) {
+          width(std::true_type{});
+          return;
+        }
+      }
+      width(std::false_type{});
+      return;
+    }
+  }
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(FSP_WG_THREADS), 0, s, static_cast<const PT*>(x.indptr),
                        static_cast<const IT*>(x.indices), static_cast<const TV*>(x.data),
@@ -361,11 +644,11 @@ static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_
   };
   if constexpr (SDD && VEC > 1) {
     if (x.n_dense % VEC != 0) {
-      launch(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, true>);
+      launch(spmm_slots_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, true>);
       return;
     }
   }
-  launch(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, false>);
+  launch(spmm_slots_kernel<T, TV, IT, PT, QT, VEC, UNROLL, PERM, OFF32, SDD, false>);
 }
 
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, bool PERM, bool SDD>
