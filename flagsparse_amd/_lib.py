@@ -206,7 +206,11 @@ def ptr(t):
 
 
 def stream_ptr(device=None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of `device` as an address.  The raw query: a
+    torch.cuda.Stream object per launch costs more than the launch's argument
+    conversion."""
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def device_arch():

@@ -23,7 +23,8 @@ The reference rebuilds its buckets with ``torch.nonzero`` on every call
 """
 
 import ctypes
-from dataclasses import dataclass
+from dataclasses import dataclass, field
+from functools import lru_cache
 
 import numpy as np
 import torch
@@ -79,12 +80,14 @@ def spmv_default_variant(x_len, elem_bytes, nnz, chunk_ok=False):
     return 0
 
 
+@lru_cache(maxsize=256)
 def spmv_config(unroll=SPMV_UNROLL, long_threshold=SPMV_LONG_THRESHOLD, seg_len=SPMV_SEG_LEN):
     lanes = (4, 8, 16, 32, 64)
     uppers = [min(l * unroll, long_threshold) for l in lanes[:-1]] + [long_threshold]
     return _dedupe(lanes, uppers, seg_len, unroll)
 
 
+@lru_cache(maxsize=1024)
 def rows_config(lanes_dense, unroll, long_threshold, seg_len, slot_scale=1):
     """SpMM / SDDMM bins for `lanes_dense` lanes along the dense dimension.
 
@@ -164,6 +167,7 @@ class CsrPlan:
     n_long_rows: int
     row_len: int = 0  # > 0: every row has exactly this many nonzeros
     indptr_base: int = 0  # indptr[0] when row_len > 0
+    _structs: dict = field(default_factory=dict, init=False, repr=False, compare=False)
 
     @property
     def bin_sizes(self):
@@ -188,6 +192,18 @@ class CsrPlan:
         region per XCD).  variant selects the SpMV loop (0 pipelined, 1 plain,
         2 plain and 3 pipelined with x staged in LDS, 4 vector chunks with x
         in LDS)."""
+        key = (max_blocks, xcd_groups, variant, self.row_len, self.indptr_base)
+        base = self._structs.get(key)
+        if base is None:
+            base = self._structs[key] = self._struct(max_blocks, xcd_groups, variant)
+        # a copy per launch: calls on other threads and streams set their own partials
+        st = _lib.FspCsrPlan.from_buffer_copy(base)
+        if partials is not None:
+            st.partials_dev = partials.data_ptr()
+            st.partials_bytes = partials.numel() * partials.element_size()
+        return st
+
+    def _struct(self, max_blocks, xcd_groups, variant):
         st = _lib.FspCsrPlan()
         st.n_bins = len(self.bin_counts)
         st.unroll = self.config.unroll
@@ -213,9 +229,6 @@ class CsrPlan:
             st.seg_end_dev = self.seg_end.data_ptr()
             st.long_rows_dev = self.long_rows.data_ptr()
             st.long_seg_ptr_dev = self.long_seg_ptr.data_ptr()
-        if partials is not None:
-            st.partials_dev = partials.data_ptr()
-            st.partials_bytes = partials.numel() * partials.element_size()
         return st
 
 

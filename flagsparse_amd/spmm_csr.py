@@ -307,6 +307,7 @@ class PreparedCsrSpmmOpt:
         "long_row_part_ptr",
         "long_row_fallback_only",
         "_handle",
+        "_described",
     )
 
     def __init__(self, data, kernel_indices, kernel_indptr, shape, n_rows, n_cols, row_lengths, max_row_nnz):
@@ -319,6 +320,7 @@ class PreparedCsrSpmmOpt:
         self.row_lengths = row_lengths
         self.max_row_nnz = int(max_row_nnz)
         self.supports_opt = data.dtype in (torch.float32, torch.float64)
+        self._described = None
         self._handle = CsrHandle(kernel_indices, kernel_indptr, self.shape)
         self.row_buckets = []
         empty = torch.empty(0, dtype=torch.int64, device=data.device)
@@ -330,7 +332,11 @@ class PreparedCsrSpmmOpt:
         self.long_row_fallback_only = False
 
     def _describe(self, plan):
-        """Fill the reference's bucket / split fields from a HIP plan."""
+        """Fill the reference's bucket / split fields from a HIP plan (once
+        per plan: a launch of the same plan has nothing to add)."""
+        if self._described is plan:
+            return
+        self._described = plan
         self.row_buckets = [
             {"kind": "rows", "slots": int(l), "max_row_nnz": int(u), "rows": int(c)}
             for l, u, c in zip(plan.config.lanes, plan.config.uppers, plan.bin_counts)

@@ -261,39 +261,29 @@ def _hip_spmv_csr_impl_prepared(prepared, x, out=None):
     """Launch fsp_spmv_csr over the prepared plan; returns y (or `out`, a
     contiguous validated result tensor the kernel writes directly).
     Replaces _triton_spmv_csr_impl_prepared (spmv_csr.py:702-746)."""
-    dtype = prepared.data.dtype
+    data, indices, indptr = prepared.data, prepared.kernel_indices, prepared.kernel_indptr
+    dtype, device = data.dtype, data.device
     require_kernel_dtype(dtype)
-    device = prepared.data.device
-    y = out if out is not None else torch.empty(prepared.n_rows, dtype=dtype, device=device)
-    if prepared.n_rows == 0:
+    n_rows, nnz, x_len = prepared.n_rows, indices.numel(), x.numel()
+    y = out if out is not None else torch.empty(n_rows, dtype=dtype, device=device)
+    if n_rows == 0:
         return y
     plan = prepared.plan()
-    acc = torch.float64 if dtype in (torch.float32, torch.float64) else torch.float32
-    partials = plan.partials(1, acc, device)
-    nnz = int(prepared.kernel_indices.numel())
-    variant = _plan.spmv_default_variant(int(x.shape[0]), x.element_size(), nnz,
-                                         _plan.chunk_aligned(prepared.kernel_indices, prepared.data))
-    st = plan.struct(partials, variant=variant)
-    _lib.check(
-        _lib.load().fsp_spmv_csr(
-            _lib.value_code(dtype),
-            _lib.index_code(prepared.kernel_indices.dtype),
-            _lib.index_code(prepared.kernel_indptr.dtype),
-            _lib.ptr(prepared.kernel_indptr),
-            _lib.ptr(prepared.kernel_indices),
-            _lib.ptr(prepared.data),
-            0,
-            None,
-            _lib.ptr(x),
-            y.data_ptr(),
-            prepared.n_rows,
-            nnz,
-            int(x.shape[0]),
-            st,
-            _lib.stream_ptr(device),
-        ),
-        "fsp_spmv_csr",
+    partials = None
+    if plan.n_segments:
+        acc = torch.float64 if dtype in (torch.float32, torch.float64) else torch.float32
+        partials = plan.partials(1, acc, device)
+    variant = 0
+    if nnz >= _plan.LDSX_MIN_NNZ:
+        variant = _plan.spmv_default_variant(x_len, x.element_size(), nnz, _plan.chunk_aligned(indices, data))
+    lib = _lib.load()
+    status = lib.fsp_spmv_csr(
+        _lib.value_code(dtype), _lib.index_code(indices.dtype), _lib.index_code(indptr.dtype), indptr.data_ptr(),
+        _lib.ptr(indices), _lib.ptr(data), 0, None, _lib.ptr(x), y.data_ptr(), n_rows, nnz, x_len,
+        plan.struct(partials, variant=variant), _lib.stream_ptr(device),
     )
+    if status:
+        _lib.check(status, "fsp_spmv_csr")
     return y
 
 
@@ -388,9 +378,10 @@ def flagsparse_spmv_csr(
     Reference: spmv_csr.py:837-945.
     """
     op_explicit = op is not None
-    op_code = _normalize_spmv_op(op, transpose=False if transpose is None else bool(transpose))
-    if op_explicit and transpose is not None and bool(transpose) != _spmv_op_transposes(op_code):
-        raise ValueError("transpose conflicts with op")
+    if op_explicit or transpose is not None or prepared is None:
+        op_code = _normalize_spmv_op(op, transpose=False if transpose is None else bool(transpose))
+        if op_explicit and transpose is not None and bool(transpose) != _spmv_op_transposes(op_code):
+            raise ValueError("transpose conflicts with op")
     if prepared is None:
         if any(arg is None for arg in (data, indices, indptr, shape)):
             raise ValueError("data, indices, indptr, and shape are required when prepared is not provided")
