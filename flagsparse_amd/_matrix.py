@@ -42,7 +42,7 @@ class CsrHandle:
     def plan(self, config):
         p = self._plans.get(config)
         if p is None:
-            p = _plan.build_plan(self.indptr, self.n_rows, config)
+            p = _plan.build_plan(self.indptr, self.n_rows, config, self.nnz)
             self._plans[config] = p
         return p
 
@@ -56,7 +56,7 @@ class CsrHandle:
         p = self._csc_plans.get(config)
         if p is None:
             colptr, _, _ = self.csc()
-            p = _plan.build_plan(colptr, self.n_cols, config)
+            p = _plan.build_plan(colptr, self.n_cols, config, self.nnz)
             self._csc_plans[config] = p
         return p
 

@@ -1,12 +1,13 @@
 """Row-length work plans for the CSR kernels (prepare-time, cached).
 
 A plan bins the rows of a CSR (or CSC) index structure by length on the GPU
-(``fsp_csr_row_bins``: a stable multi-split, rows stay ascending inside a
-bin) and cuts rows longer than the last bin into nnz-balanced segments.  The
-kernels then run every bin and every segment in one launch; rows that were
-split get a second, deterministic pass that adds their segment partials in
-order.  Building a plan costs one device->host copy of the bin boundaries and
-of the long rows' extents; running with a plan costs no host sync.
+(a stable multi-split, rows stay ascending inside a bin) and cuts rows longer
+than the last bin into nnz-balanced segments, both in ``fsp_csr_build_plan``.
+The kernels then run every bin and every segment in one launch; rows that
+were split get a second, deterministic pass that adds their segment partials
+in order.  Building a plan costs one device->host copy, of the validation
+figures, the bin boundaries and the number of segments; running with a plan
+costs no host sync.
 
 Bin layouts per kernel family (``unroll`` = nonzeros per lane per trip):
 
@@ -26,7 +27,6 @@ import ctypes
 from dataclasses import dataclass, field
 from functools import lru_cache
 
-import numpy as np
 import torch
 
 from . import _lib
@@ -232,25 +232,53 @@ class CsrPlan:
         return st
 
 
-def _launch_row_bins(indptr, n_rows, config, offsets):
-    """Launch the row binning of `indptr` (device tensor, int32/int64) into
-    `offsets` (device int64[n_bins + 1]); returns the row-id buffer."""
+_N_STATS = 6  # figures ahead of the bin offsets in fsp_csr_build_plan's meta
+_KEEP_BYTES = 1 << 20
+
+
+def _build(indptr, indices, n_rows, nnz, config):
+    """fsp_csr_build_plan and the one host readback: (figures, plan arrays).
+    The plan arrays are None without `config`; they are usable only if the
+    figures describe a valid CSR of at most nnz nonzeros."""
     device = indptr.device
-    nb = len(config.uppers) + 1  # regular bins + the long bin
     lib = _lib.load()
-    rows = torch.empty(max(1, n_rows), dtype=torch.int32, device=device)
+    n_bins = len(config.uppers) + 1 if config is not None else 0  # regular bins + the long bin
+    n_meta = _N_STATS + (n_bins + 2 if n_bins else 0)
     ws_bytes = ctypes.c_int64(0)
-    _lib.check(lib.fsp_csr_row_bins_workspace(n_rows, nb, ctypes.byref(ws_bytes)), "fsp_csr_row_bins_workspace")
-    ws = torch.empty(max(1, ws_bytes.value), dtype=torch.uint8, device=device)
-    uppers = (ctypes.c_int64 * nb)(*[int(u) for u in config.uppers], 0)
+    _lib.check(lib.fsp_csr_build_plan_workspace(n_rows, nnz, n_bins, ctypes.byref(ws_bytes)),
+               "fsp_csr_build_plan_workspace")
+    max_long = max_seg = 0
+    uppers, seg_len, buf32 = None, 1, None
+    if n_bins:
+        seg_len = config.seg_len
+        max_long = min(n_rows, nnz // (config.uppers[-1] + 1))
+        max_seg = max_long + nnz // seg_len if max_long else 0
+        uppers = (ctypes.c_int64 * n_bins)(*config.uppers, 0)
+        buf32 = torch.empty(n_rows + max_seg, dtype=torch.int32, device=device)
+    # int64 words: meta | segment begins | segment ends | segment ranges | workspace
+    o_end, o_ptr = n_meta + max_seg, n_meta + 2 * max_seg
+    o_ws = o_ptr + (max_long + 1 if max_long else 0)
+    buf = torch.empty(o_ws + -(-ws_bytes.value // 8), dtype=torch.int64, device=device)
+    at64, at32 = buf.data_ptr(), (buf32.data_ptr() if buf32 is not None else 0)
     _lib.check(
-        lib.fsp_csr_row_bins(
-            _index_code(indptr), _lib.ptr(indptr), n_rows, nb, uppers, rows.data_ptr(),
-            offsets.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_ptr(device),
+        lib.fsp_csr_build_plan(
+            _index_code(indptr), indptr.data_ptr(), 0 if indices is None else _index_code(indices),
+            None if indices is None else _lib.ptr(indices), n_rows, nnz, n_bins, uppers, seg_len, at64, at32, max_seg,
+            at32 + 4 * n_rows, at64 + 8 * n_meta, at64 + 8 * o_end, max_long, at64 + 8 * o_ptr, at64 + 8 * o_ws,
+            ws_bytes.value, _lib.stream_ptr(device),
         ),
-        "fsp_csr_row_bins",
+        "fsp_csr_build_plan",
     )
-    return rows
+    host = buf[:n_meta].tolist()  # the one host sync
+    if not n_bins:
+        return host, None
+    off, n_seg = host[_N_STATS:-1], host[-1]
+    n_long = off[n_bins] - off[n_bins - 1]
+    segments = None
+    if 0 < n_long <= max_long and 0 < n_seg <= max_seg:
+        segments = (buf32[n_rows:n_rows + n_seg], buf[n_meta:n_meta + n_seg], buf[o_end:o_end + n_seg],
+                    buf[o_ptr:o_ptr + n_long + 1], n_seg)
+    return host, (buf32[:n_rows], off, segments)
 
 
 def _row_len_if_constant(n_rows, first, last, max_len):
@@ -261,23 +289,16 @@ def _row_len_if_constant(n_rows, first, last, max_len):
     return 0
 
 
-def build_plan(indptr, n_rows, config):
-    """Bin the rows described by `indptr` (device tensor, int32/int64)."""
+def build_plan(indptr, n_rows, config, nnz=None):
+    """Bin the rows described by `indptr` (device tensor, int32/int64).  nnz:
+    an upper bound on their nonzeros (read from indptr when not given)."""
     n_rows = int(n_rows)
-    nb = len(config.uppers) + 1
-    meta = torch.empty(nb + 1 + 3, dtype=torch.int64, device=indptr.device)
-    rows = _launch_row_bins(indptr, n_rows, config, meta[: nb + 1])
-    if n_rows > 0:
-        ip = indptr[: n_rows + 1]
-        meta[nb + 1] = ip[0]
-        meta[nb + 2] = ip[n_rows]
-        meta[nb + 3] = (ip[1:] - ip[:-1]).max()
-    else:
-        meta[nb + 1:] = 0
-    host = meta.cpu().tolist()  # host sync (prepare time only)
-    first, last, max_len = host[nb + 1:]
-    return _finish_plan(indptr, n_rows, config, rows, host[: nb + 1],
-                        _row_len_if_constant(n_rows, first, last, max_len), first)
+    if nnz is None:
+        ends = indptr[:n_rows + 1:max(1, n_rows)].tolist()
+        nnz = max(0, ends[-1] - ends[0])
+    host, arrays = _build(indptr, None, n_rows, int(nnz), config)
+    first, last, max_len = host[0], host[1], host[5]
+    return _finish_plan(indptr, n_rows, config, arrays, _row_len_if_constant(n_rows, first, last, max_len), first)
 
 
 def inspect_csr(indptr, indices, n_rows, nnz, config=None):
@@ -286,19 +307,8 @@ def inspect_csr(indptr, indices, n_rows, nnz, config=None):
     indptr_last, n_decreasing, min_col, max_col (None without nonzeros) and
     max_row; plan is None without `config` or when the row pointer is not a
     valid CSR (the caller raises on the stats first)."""
-    device = indptr.device
     n_rows, nnz = int(n_rows), int(nnz)
-    nb = len(config.uppers) + 1 if config is not None else 0
-    meta = torch.empty(6 + (nb + 1 if config is not None else 0), dtype=torch.int64, device=device)
-    _lib.check(
-        _lib.load().fsp_csr_inspect(
-            _index_code(indptr), _lib.ptr(indptr), _index_code(indices), _lib.ptr(indices) if nnz else None,
-            n_rows, nnz, meta.data_ptr(), _lib.stream_ptr(device),
-        ),
-        "fsp_csr_inspect",
-    )
-    rows = _launch_row_bins(indptr, n_rows, config, meta[6:]) if config is not None else None
-    host = meta.cpu().tolist()  # the one host sync
+    host, arrays = _build(indptr, indices, n_rows, nnz, config)
     stats = {
         "indptr_first": host[0],
         "indptr_last": host[1],
@@ -309,16 +319,17 @@ def inspect_csr(indptr, indices, n_rows, nnz, config=None):
     }
     plan = None
     if config is not None and host[0] == 0 and host[1] == nnz and host[2] == 0:
-        plan = _finish_plan(indptr, n_rows, config, rows, host[6:],
+        plan = _finish_plan(indptr, n_rows, config, arrays,
                             _row_len_if_constant(n_rows, host[0], host[1], stats["max_row"]), host[0])
     return stats, plan
 
 
-def _finish_plan(indptr, n_rows, config, rows, off, row_len=0, indptr_base=0):
-    """The plan from the bin offsets `off` (host list) of a valid CSR.
+def _finish_plan(indptr, n_rows, config, arrays, row_len=0, indptr_base=0):
+    """The plan from the arrays of _build for a valid CSR.
     row_len > 0 (every row that long, indptr[i] = indptr_base + i * row_len)
     is kept for a single-bin plan: its kernels then compute row bounds."""
     device = indptr.device
+    rows, off, segments = arrays
     nb = len(config.uppers) + 1
     counts = [off[i + 1] - off[i] for i in range(nb)]
     regular = counts[:-1]
@@ -327,39 +338,28 @@ def _finish_plan(indptr, n_rows, config, rows, off, row_len=0, indptr_base=0):
     if identity and n_rows:
         # one non-empty regular bin holding every row, in order: drop the list
         regular = [n_rows if c else 0 for c in regular]
-    empty_i32 = torch.empty(0, dtype=torch.int32, device=device)
-    empty_i64 = torch.empty(0, dtype=torch.int64, device=device)
-    seg_row = seg_begin = seg_end = long_seg_ptr = empty_i64
-    long_rows = empty_i32
     n_seg = 0
-    if n_long:
-        long_rows = rows[off[nb - 1]: off[nb]].clone()
-        lr = long_rows.to(torch.int64)
-        ip = indptr.to(torch.int64)
-        host = torch.stack([lr, ip[lr], ip[lr + 1]]).cpu().numpy()  # one readback
-        host_rows, starts, ends = host[0].astype(np.int32), host[1], host[2]
-        lens = ends - starts
-        seg_len = config.seg_len
-        nseg = (lens + seg_len - 1) // seg_len
-        ptr = np.zeros(n_long + 1, dtype=np.int64)
-        np.cumsum(nseg, out=ptr[1:])
-        n_seg = int(ptr[-1])
-        owner = np.repeat(np.arange(n_long, dtype=np.int64), nseg)
-        j = np.arange(n_seg, dtype=np.int64) - ptr[owner]
-        # even split: segment j of a row covers [len*j/n, len*(j+1)/n)
-        b = starts[owner] + (lens[owner] * j) // nseg[owner]
-        e = starts[owner] + (lens[owner] * (j + 1)) // nseg[owner]
-        seg_row = torch.from_numpy(host_rows[owner].copy()).to(device)
-        seg_begin = torch.from_numpy(b).to(device)
-        seg_end = torch.from_numpy(e).to(device)
-        long_seg_ptr = torch.from_numpy(ptr).to(device)
+    if segments is not None:
+        seg_row, seg_begin, seg_end, long_seg_ptr, n_seg = segments
+        long_rows = rows[off[nb - 1]: off[nb]]
+        held = seg_begin.untyped_storage().nbytes()
+        if held > _KEEP_BYTES and held > 8 * 8 * n_seg:  # few segments of what was provided for
+            rows, seg_row, long_rows = rows.clone(), seg_row.clone(), long_rows.clone()
+            seg_begin, seg_end, long_seg_ptr = seg_begin.clone(), seg_end.clone(), long_seg_ptr.clone()
+    else:
+        if n_long:
+            raise RuntimeError("the row pointer holds more nonzeros than the plan was built for")
+        seg_row = long_rows = torch.empty(0, dtype=torch.int32, device=device)
+        seg_begin = seg_end = long_seg_ptr = torch.empty(0, dtype=torch.int64, device=device)
+        if rows.untyped_storage().nbytes() > 4 * n_rows + _KEEP_BYTES:
+            rows = rows.clone()
     return CsrPlan(
         config=config,
         n_rows=n_rows,
         rows=rows,
         bin_counts=regular,
         identity=bool(identity),
-        seg_row=seg_row if n_seg else empty_i32,
+        seg_row=seg_row,
         seg_begin=seg_begin,
         seg_end=seg_end,
         long_rows=long_rows,

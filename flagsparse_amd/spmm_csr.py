@@ -65,10 +65,11 @@ def _prepare_spmm_csr_matrix(data, indices, indptr, shape):
     return _inspect_spmm_csr_matrix(data, indices, indptr, shape)[0]
 
 
-def _inspect_spmm_csr_matrix(data, indices, indptr, shape, plan_config=None):
+def _inspect_spmm_csr_matrix(data, indices, indptr, shape, plan_config=None, row_lengths=True):
     """_prepare_spmm_csr_matrix plus, with `plan_config`, the row-bin plan,
     from one device inspection and ONE host readback.  Returns (validated
-    tuple, plan or None)."""
+    tuple, plan or None); row_lengths=False leaves the tuple's row lengths
+    None for callers that do not keep them."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
     if data.ndim != 1 or indices.ndim != 1 or indptr.ndim != 1:
@@ -106,7 +107,10 @@ def _inspect_spmm_csr_matrix(data, indices, indptr, shape, plan_config=None):
             raise IndexError("indices out of range for n_cols")
         if stats["max_col"] > _INDEX_LIMIT_INT32:
             raise ValueError("column indices exceed the int32 range supported by the SpMM kernel")
-    row_lengths = indptr[1:] - indptr[:-1] if n_rows > 0 else indptr.new_empty((0,))
+    if not row_lengths:
+        row_lengths = None
+    else:
+        row_lengths = indptr[1:] - indptr[:-1] if n_rows > 0 else indptr.new_empty((0,))
     return (data, indices, indptr, n_rows, n_cols, row_lengths, stats["max_row"]), plan
 
 
@@ -219,7 +223,7 @@ def flagsparse_spmm_csr(
     if not transposes and torch.is_tensor(B) and B.ndim == 2 and data.dtype in KERNEL_VALUE_DTYPES:
         plan_cfg = _base_plan_config(int(B.shape[1]), data.element_size(), block_n, block_nnz)
     (data, indices, indptr, n_rows, n_cols, row_lengths, max_row_nnz), plan = _inspect_spmm_csr_matrix(
-        data, indices, indptr, shape, plan_cfg
+        data, indices, indptr, shape, plan_cfg, row_lengths=False
     )
     if B.ndim != 2:
         raise ValueError("B must be a 2D dense tensor")

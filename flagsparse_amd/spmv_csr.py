@@ -119,7 +119,8 @@ class PreparedCsrSpmv:
     def plan(self, config=None):
         """The row-bin plan of this matrix (built on first use, then cached)."""
         if self._plan is None or (config is not None and self._plan.config != config):
-            self._plan = _plan.build_plan(self.kernel_indptr, self.n_rows, config or _plan.spmv_config())
+            self._plan = _plan.build_plan(self.kernel_indptr, self.n_rows, config or _plan.spmv_config(),
+                                          self.kernel_indices.numel())
         return self._plan
 
 

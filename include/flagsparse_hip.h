@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FSP_ABI_VERSION 16
+#define FSP_ABI_VERSION 17
 #define FSP_MAX_BINS 8
 
 typedef enum fsp_value_type {
@@ -59,8 +59,7 @@ typedef struct fsp_bin {
 
 /* Work plan of one CSR (or CSC) matrix: rows binned by length, plus the
  * nnz-balanced split of rows longer than the last bin into segments.  All
- * arrays are device memory owned by the caller (built by fsp_csr_row_bins and
- * the host-side segment split). */
+ * arrays are device memory owned by the caller (built by fsp_csr_build_plan). */
 typedef struct fsp_csr_plan {
   int32_t n_bins;
   int32_t unroll;                 /* nonzeros per lane per loop trip (1..8) */
@@ -129,6 +128,28 @@ int fsp_csr_row_bins(int32_t indptr_type, const void* indptr_dev, int64_t n_rows
                      int32_t n_bins, const int64_t* upper,
                      int32_t* rows_out_dev, int64_t* bin_offsets_out_dev,
                      void* ws_dev, int64_t ws_bytes, void* stream);
+
+/* fsp_csr_inspect, fsp_csr_row_bins and the segment split of the rows in the
+ * last bin, in one call whose results the host reads back once.
+ *   meta[6 + n_bins + 2]: the six figures of fsp_csr_inspect (column figures
+ *   INT64_MAX / INT64_MIN without indices), the n_bins + 1 bin offsets and the
+ *   number of segments; n_bins 0 gives the figures alone (meta[6]).
+ *   rows[n_rows]: row ids by bin, as fsp_csr_row_bins.
+ *   A row of the last bin is cut evenly into ceil(len / seg_len) segments:
+ *   seg_row / seg_begin / seg_end [max_segments] and long_seg_ptr
+ *   [max_long + 1] (segment range per such row, in the order of rows).
+ * max_long >= the rows of the last bin and max_segments >= their segments for
+ * a valid CSR; an invalid one (the figures tell) leaves the plan arrays with
+ * unspecified contents, and nothing is written past either bound.  Nothing
+ * here trusts the structure.  indices may be NULL (no column figures). */
+int fsp_csr_build_plan_workspace(int64_t n_rows, int64_t nnz, int32_t n_bins, int64_t* bytes);
+int fsp_csr_build_plan(int32_t indptr_type, const void* indptr_dev, int32_t index_type,
+                       const void* indices_dev, int64_t n_rows, int64_t nnz,
+                       int32_t n_bins, const int64_t* upper, int64_t seg_len,
+                       int64_t* meta_dev, int32_t* rows_dev, int64_t max_segments,
+                       int32_t* seg_row_dev, int64_t* seg_begin_dev, int64_t* seg_end_dev,
+                       int64_t max_long, int64_t* long_seg_ptr_dev,
+                       void* ws_dev, int64_t ws_bytes, void* stream);
 
 /* ---- CSR -> CSC -----------------------------------------------------------
  * Replaces _transpose_csr_for_spmv (spmv_csr.py:498-536) and
