@@ -25,6 +25,27 @@ def _acc_dtype(dtype):
     return torch.float64 if dtype == torch.float64 else torch.float32
 
 
+# Half of one XCD's 4 MiB L2: values up to this size stay there beside the dense
+# rows, see _permuted_in_kernel.
+_PERMUTED_BYTES = 2 << 20
+
+
+def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes):
+    """True where the transposed kernels read data[perm[q]] beside their
+    gathers of the dense rows (ld x rows) instead of after a pass that gathers
+    the values: where the kernel's lanes share their nonzeros (the conditions
+    of csrc/spmm_kernels.hpp; elsewhere every lane would read it for itself)
+    and the values stay in the L2s.  Graphs of mean degree 14, N = 64, f32:
+    16000 nodes (0.9 MB of values) 15.1 against 20.9 us, 32000 nodes 19.6
+    against 22.1, 64000 nodes (3.6 MB) 37.0 against 35.3, 128000 nodes 78 against
+    68, where each of those reads is another 128 bytes across the fabric."""
+    elem = data.element_size()
+    dense = rows * ld * elem
+    return (perm.numel() * elem <= _PERMUTED_BYTES and lanes >= 4 and n_dense >= 16 // elem
+            and perm.dtype == torch.int32 and dense + ld * elem < 1 << 32 and n_out * n_dense * elem < 1 << 32
+            and (lanes < 16 or dense < 64 << 20))
+
+
 class CsrHandle:
     __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "_plans", "_csc", "_csc_plans")
 
@@ -66,12 +87,13 @@ class CsrHandle:
         """C = A B (transpose=False) or A^T B (transpose=True); B row-major.
         max_blocks > 0: persistent launch of at most that many workgroups;
         xcd_groups > 1: XCD-region tile mapping (see _plan.CsrPlan.struct).
-        transpose: the values are first gathered into CSC order (one pass of
-        nnz random reads); the kernel then streams them like a plain CSR.  A
-        kernel that loads data[perm[q]] itself puts that random read in every
-        nonzero's dependent chain and measures 10-19 % slower (262144^2 power
-        law at N = 64 and the 200000-node graph at N = 128, f32 and bf16).
-        values_via_perm=True keeps that form; both are bitwise equal.
+        transpose: the kernel reads data[perm[q]] itself where one lane does
+        so for its whole group (_permuted_in_kernel).  Elsewhere the values are
+        first gathered into CSC order (one pass of nnz random reads) and
+        streamed like a plain CSR's: with every lane of a group reading
+        data[perm[q]] in its own dependent chain the product measures 10-19 %
+        slower (262144^2 power law, N = 64).  values_via_perm=True reads through
+        perm in any case; all forms are bitwise equal.
         data may be wider than B (float64 values over float32 operands,
         float32 over 16-bit ones): the sums are kept in data's dtype and C, in
         B's dtype, is rounded once."""
@@ -90,7 +112,8 @@ class CsrHandle:
             colptr, rowind, perm = self.csc()
             plan = self.csc_plan(cfg)
             ptr_t, idx_t, perm_t = colptr, rowind, perm
-            if not values_via_perm:
+            if not values_via_perm and (data.dtype != B.dtype or not _permuted_in_kernel(
+                    data, perm, int(B.stride(0)), int(B.shape[0]), n_out, n_dense, G)):
                 data, perm_t = gather_values(data, perm), None
         else:
             plan = self.plan(cfg)
@@ -153,17 +176,21 @@ class CsrHandle:
         cfg = _plan.spmm_config(G)
         colptr, rowind, perm = self.csc()
         plan = self.csc_plan(cfg)
-        data_t = gather_values(data, perm) if self.nnz else data
+        name = "fsp_spmm_csr_trans_sddmm"
+        if self.nnz and not _permuted_in_kernel(data, perm, int(dC.stride(0)), self.n_rows, self.n_cols, n_dense, G):
+            data = gather_values(data, perm)
+        elif self.nnz:
+            name = "fsp_spmm_csr_trans_sddmm_perm"
         partials = plan.partials(n_dense, _acc_dtype(data.dtype), device)
         st = plan.struct(partials)
         _lib.check(
-            _lib.load().fsp_spmm_csr_trans_sddmm(
+            getattr(_lib.load(), name)(
                 _lib.value_code(data.dtype), _lib.index_code(rowind.dtype), _lib.index_code(colptr.dtype),
-                _lib.ptr(colptr), _lib.ptr(rowind), _lib.ptr(data_t), _lib.index_code(perm.dtype), _lib.ptr(perm),
+                _lib.ptr(colptr), _lib.ptr(rowind), _lib.ptr(data), _lib.index_code(perm.dtype), _lib.ptr(perm),
                 dC.data_ptr(), int(dC.stride(0)), B.data_ptr(), int(B.stride(0)), dB.data_ptr(), int(dB.stride(0)),
                 dvalues.data_ptr(), self.n_cols, n_dense, self.nnz, self.n_rows, G, st, _lib.stream_ptr(device),
             ),
-            "fsp_spmm_csr_trans_sddmm",
+            name,
         )
         return dB, dvalues
 

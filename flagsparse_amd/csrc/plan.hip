@@ -157,14 +157,31 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void fill_i64_kernel(int64_t* __res
 
 template <int BYTES> struct blob { alignas(BYTES < 16 ? BYTES : 16) unsigned char b[BYTES]; };
 
+// out[q] = in[perm[q]].  Each thread moves kGatherItems consecutive elements:
+// its permutation entries come as whole vectors, its reads of `in` are all in
+// flight together and its results leave as vectors.  The reads are what
+// bounds it: each is a cache line of its own, 2.5-2.8 clocks per line and CU
+// from L2 (2.8 M values of 2 bytes: 21.8 us
+// with one element per thread, 18.0 us with four, 19.4 with eight).
+constexpr int kGatherItems = 4;
 template <int BYTES, typename QT>
 __global__ __launch_bounds__(FSP_WG_THREADS) void gather_kernel(
     const QT* __restrict__ perm, const blob<BYTES>* __restrict__ in, blob<BYTES>* __restrict__ out,
     int64_t n) {
-  for (int64_t q = static_cast<int64_t>(blockIdx.x) * FSP_WG_THREADS + threadIdx.x; q < n;
-       q += static_cast<int64_t>(gridDim.x) * FSP_WG_THREADS) {
-    out[q] = in[static_cast<int64_t>(perm[q])];
+  struct perms { QT q[kGatherItems]; };
+  struct items { blob<BYTES> v[kGatherItems]; };
+  const int64_t whole = n / kGatherItems;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * FSP_WG_THREADS;
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * FSP_WG_THREADS + threadIdx.x;
+  for (int64_t i = tid; i < whole; i += stride) {
+    const perms p = *reinterpret_cast<const perms*>(perm + i * kGatherItems);
+    items o;
+#pragma unroll
+    for (int k = 0; k < kGatherItems; ++k) o.v[k] = in[static_cast<int64_t>(p.q[k])];
+    *reinterpret_cast<items*>(out + i * kGatherItems) = o;
   }
+  const int64_t q = whole * kGatherItems + tid;
+  if (q < n) out[q] = in[static_cast<int64_t>(perm[q])];
 }
 
 static inline int grid_for(int64_t n) {
@@ -289,7 +306,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void csr_stats_kernel(const PT* __r
 
 template <typename QT>
 static int launch_gather(int32_t elem_bytes, const QT* perm, const void* in, void* out, int64_t n, hipStream_t s) {
-  const dim3 grid(grid_for(n)), block(FSP_WG_THREADS);
+  const dim3 grid(grid_for(ceil_div(n, int64_t(kGatherItems)))), block(FSP_WG_THREADS);
   switch (elem_bytes) {
     case 1: hipLaunchKernelGGL((gather_kernel<1, QT>), grid, block, 0, s, perm, static_cast<const blob<1>*>(in), static_cast<blob<1>*>(out), n); break;
     case 2: hipLaunchKernelGGL((gather_kernel<2, QT>), grid, block, 0, s, perm, static_cast<const blob<2>*>(in), static_cast<blob<2>*>(out), n); break;

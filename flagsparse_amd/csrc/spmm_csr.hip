@@ -120,18 +120,21 @@ extern "C" int fsp_spmm_csr_wide(int32_t dense_type, int32_t index_type, int32_t
                     C_dev, ldc, n_rows, n_dense, nnz, b_rows, lanes_n, plan, stream, true);
 }
 
-extern "C" int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, int32_t indptr_type,
-                                        const void* colptr_dev, const void* rowind_dev, const void* data_csc_dev,
-                                        int32_t pos_type, const void* pos_dev, const void* dC_dev, int64_t lddc,
-                                        const void* B_dev, int64_t ldb, void* dB_dev, int64_t lddb,
-                                        void* dvalues_dev, int64_t n_cols, int64_t n_dense, int64_t nnz,
-                                        int64_t n_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream) {
+namespace fsp {
+
+// data_dev in CSC order, or (csr_values) in CSR order and read through pos.
+static int trans_sddmm_entry(bool csr_values, int32_t value_type, int32_t index_type, int32_t indptr_type,
+                             const void* colptr_dev, const void* rowind_dev, const void* data_dev,
+                             int32_t pos_type, const void* pos_dev, const void* dC_dev, int64_t lddc,
+                             const void* B_dev, int64_t ldb, void* dB_dev, int64_t lddb,
+                             void* dvalues_dev, int64_t n_cols, int64_t n_dense, int64_t nnz,
+                             int64_t n_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream) {
   if (n_cols < 0 || n_dense < 0 || nnz < 0 || n_rows < 0) {
     return fail(FSP_ERR_ARG, "fsp_spmm_csr_trans_sddmm: negative size");
   }
   int st = check_plan(plan, n_cols);
   if (st) return st;
-  if (colptr_dev == nullptr || (nnz > 0 && (rowind_dev == nullptr || data_csc_dev == nullptr || pos_dev == nullptr ||
+  if (colptr_dev == nullptr || (nnz > 0 && (rowind_dev == nullptr || data_dev == nullptr || pos_dev == nullptr ||
                                             dvalues_dev == nullptr || dC_dev == nullptr || B_dev == nullptr)) ||
       (n_cols > 0 && n_dense > 0 && dB_dev == nullptr)) {
     return fail(FSP_ERR_ARG, "fsp_spmm_csr_trans_sddmm: NULL pointer");
@@ -162,7 +165,7 @@ extern "C" int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, 
     });
   }
   if (n_cols == 0) return FSP_OK;  // nnz > 0 needs columns: unreachable for a valid CSC
-  spmm_args x{colptr_dev, rowind_dev, data_csc_dev, nullptr, dC_dev, lddc, dB_dev, lddb, n_cols, n_dense, lanes_n,
+  spmm_args x{colptr_dev, rowind_dev, data_dev, csr_values ? pos_dev : nullptr, dC_dev, lddc, dB_dev, lddb, n_cols, n_dense, lanes_n,
               nnz, n_rows};
   x.Bj = B_dev;
   x.ldbj = ldb;
@@ -170,6 +173,31 @@ extern "C" int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, 
   x.dvals = dvalues_dev;
   FSP_DISPATCH_VALUE(value_type, T, { return spmm_sdd_launch<T>(index_type, indptr_type, pos_type, x, plan, s); });
   return FSP_OK;
+}
+
+}  // namespace fsp
+
+extern "C" int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, int32_t indptr_type,
+                                        const void* colptr_dev, const void* rowind_dev, const void* data_csc_dev,
+                                        int32_t pos_type, const void* pos_dev, const void* dC_dev, int64_t lddc,
+                                        const void* B_dev, int64_t ldb, void* dB_dev, int64_t lddb,
+                                        void* dvalues_dev, int64_t n_cols, int64_t n_dense, int64_t nnz,
+                                        int64_t n_rows, int32_t lanes_n, const fsp_csr_plan* plan, void* stream) {
+  return trans_sddmm_entry(false, value_type, index_type, indptr_type, colptr_dev, rowind_dev, data_csc_dev, pos_type,
+                           pos_dev, dC_dev, lddc, B_dev, ldb, dB_dev, lddb, dvalues_dev, n_cols, n_dense, nnz, n_rows,
+                           lanes_n, plan, stream);
+}
+
+extern "C" int fsp_spmm_csr_trans_sddmm_perm(int32_t value_type, int32_t index_type, int32_t indptr_type,
+                                             const void* colptr_dev, const void* rowind_dev, const void* data_dev,
+                                             int32_t pos_type, const void* pos_dev, const void* dC_dev, int64_t lddc,
+                                             const void* B_dev, int64_t ldb, void* dB_dev, int64_t lddb,
+                                             void* dvalues_dev, int64_t n_cols, int64_t n_dense, int64_t nnz,
+                                             int64_t n_rows, int32_t lanes_n, const fsp_csr_plan* plan,
+                                             void* stream) {
+  return trans_sddmm_entry(true, value_type, index_type, indptr_type, colptr_dev, rowind_dev, data_dev, pos_type,
+                           pos_dev, dC_dev, lddc, B_dev, ldb, dB_dev, lddb, dvalues_dev, n_cols, n_dense, nnz, n_rows,
+                           lanes_n, plan, stream);
 }
 
 extern "C" int fsp_spmm_csr_noalloc(int32_t value_type, int32_t index_type, int32_t indptr_type,

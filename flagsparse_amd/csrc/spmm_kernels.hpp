@@ -339,8 +339,8 @@ constexpr int kMinBlocks = SDD ? 5 : (UNROLL > 4 ? 6 : 8);
 // loads from 6.1 to 2.6 million (262144^2, N = 64).  100003 x 70001 f64,
 // N = 75: 290 -> 242 us; 1024-matrix batch, N = 32: 686 -> 664 us;
 // 200000-node graph, bf16 N = 128: 89 -> 86 us, its backward 144 -> 141 us.
-template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool SDD,
-          bool TAIL>
+template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool PERM,
+          bool SDD, bool TAIL>
 __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spmm_bins_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
     const T* __restrict__ B, int64_t ldb, uint32_t b_bytes, T* __restrict__ C, int64_t ldc, int64_t n_dense, uint32_t nnz,
@@ -410,8 +410,8 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spm
       const P q = p + (static_cast<P>(r * LANES + ql) << s_log2);
       const O at = q < end ? static_cast<O>(q) : kAbsent;
       c[r] = indices_b.load(at);
-      a[r] = data_b.load(at);
-      if constexpr (SDD) pq[r] = pos_b.load(at);
+      if constexpr (!PERM) a[r] = data_b.load(at);
+      if constexpr (PERM || SDD) pq[r] = pos_b.load(at);
     }
   };
 
@@ -453,7 +453,8 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spm
       for (int r = 0; r < kRegs; ++r) {
         const bool ok = p + (static_cast<P>(r * LANES + ql) << s_log2) < end;
         off[r] = ok ? static_cast<O>(c[r]) * row_bytes : outside;
-        av[r] = static_cast<A>(a[r]);
+        // the permuted value's random read runs beside the B rows' gathers
+        if constexpr (PERM) a[r] = data_b.load(ok ? static_cast<O>(pq[r]) : kAbsent);
       }
       const P pn = p + (static_cast<P>(kTrip) << s_log2);
       const bool same = pn < end;
@@ -475,6 +476,10 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spm
         // a branch the compiler could not count the loads in flight, and the
         // last B row of the batch would wait for the prefetch too.
         if constexpr (u0 == 0) trip(same ? pn : beg_n + slot, same ? end : end_n, cn, an, pqn);
+        if constexpr (u0 == 0) {
+#pragma unroll
+          for (int r = 0; r < kRegs; ++r) av[r] = static_cast<A>(a[r]);
+        }
         static_for<UNROLL>([&](auto u) {
           constexpr int n = u0 + decltype(u)::value;
           const A x = bcast<LANES, n % LANES>(av[n / LANES]);
@@ -508,8 +513,8 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spm
 #pragma unroll
       for (int r = 0; r < kRegs; ++r) {
         c[r] = cn[r];
-        a[r] = an[r];
-        if constexpr (SDD) pq[r] = pqn[r];
+        if constexpr (!PERM) a[r] = an[r];
+        if constexpr (PERM || SDD) pq[r] = pqn[r];
       }
       p = pn;
       prefetched = true;
@@ -602,13 +607,12 @@ template <typename T, typename TV, typename IT, typename PT, typename QT, int VE
           bool SDD>
 static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_of<TV>::type* partials,
                         const launch_table& tab, hipStream_t s) {
-  const sdd_args<T, QT> sd{static_cast<const T*>(x.Bj), x.ldbj, static_cast<const QT*>(x.pos),
+  const sdd_args<T, QT> sd{static_cast<const T*>(x.Bj), x.ldbj, static_cast<const QT*>(SDD ? x.pos : x.perm),
                            static_cast<T*>(x.dvals)};
   // Groups of 4 or more lanes of whole vectors share their nonzeros through
-  // broadcasts; narrower groups, and values read through a permutation, load
-  // them per lane.
+  // broadcasts; narrower groups load them per lane.
   const int64_t b_bytes = x.b_rows * x.ldb * (int64_t)sizeof(T);
-  if constexpr (VEC > 1 && !PERM && OFF32) {
+  if constexpr (VEC > 1 && OFF32) {
     const auto bins = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(FSP_WG_THREADS), 0, s, static_cast<const PT*>(x.indptr),
                          static_cast<const IT*>(x.indices), static_cast<const TV*>(x.data),
@@ -618,9 +622,9 @@ static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_
     const auto width = [&](auto tail) {
       constexpr bool TAIL = decltype(tail)::value;
       if (g_log2 >= 4) {
-        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 16, SDD, TAIL>);
+        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 16, PERM, SDD, TAIL>);
       } else {
-        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 4, SDD, TAIL>);
+        bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 4, PERM, SDD, TAIL>);
       }
     };
     // (b_bytes + a row stays below the offset that marks an absent nonzero)
@@ -683,9 +687,11 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
     // 32-bit byte offsets when every array the kernel addresses fits in 4 GiB,
     // whatever the row pointer's type (its values fit then too).  With 64-bit
     // pointers and 64-bit offsets the f64 N = 75 product above took 301 us
-    // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.
+    // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.  Groups of one
+    // or two lanes are the other way round (104608-node graph, int64 indices,
+    // f32 N = 8: 28.7 us with 64-bit offsets, 29.6 us with 32-bit ones).
     const int64_t lim = int64_t(1) << 32;
-    const bool off32 = (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
+    const bool off32 = (std::is_same<PT, int32_t>::value || G >= 4) && (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
                        x.nnz * (int64_t)sizeof(TV) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
                        x.nnz * (int64_t)sizeof(QT) < lim && x.b_rows * x.ldb * (int64_t)sizeof(T) < lim &&
                        x.n_rows * x.ldc * (int64_t)sizeof(T) < lim && partial_bytes < lim &&
@@ -746,7 +752,10 @@ int spmm_sdd_launch(int32_t index_type, int32_t indptr_type, int32_t pos_type, c
                     const fsp_csr_plan* plan, hipStream_t s) {
   FSP_DISPATCH_INDEX(index_type, IT, {
     FSP_DISPATCH_INDEX(indptr_type, PT, {
-      FSP_DISPATCH_INDEX(pos_type, QT, { return launch_spmm_vec<T, T, IT, PT, QT, false, true>(x, plan, s); });
+      FSP_DISPATCH_INDEX(pos_type, QT, {
+        if (x.perm != nullptr) return launch_spmm_vec<T, T, IT, PT, QT, true, true>(x, plan, s);
+        return launch_spmm_vec<T, T, IT, PT, QT, false, true>(x, plan, s);
+      });
     });
   });
   return FSP_OK;

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FSP_ABI_VERSION 17
+#define FSP_ABI_VERSION 18
 #define FSP_MAX_BINS 8
 
 typedef enum fsp_value_type {
@@ -265,6 +265,17 @@ int fsp_spmm_csr_trans_sddmm(int32_t value_type, int32_t index_type, int32_t ind
                              void* dB_dev, int64_t lddb, void* dvalues_dev,
                              int64_t n_cols, int64_t n_dense, int64_t nnz, int64_t n_rows,
                              int32_t lanes_n, const fsp_csr_plan* plan, void* stream);
+
+/* fsp_spmm_csr_trans_sddmm with the values in CSR order: CSC nonzero q has the
+ * value data[pos[q]], read inside the kernel beside the gathers of dC.  Same
+ * results, without the caller's pass over the values (fsp_gather). */
+int fsp_spmm_csr_trans_sddmm_perm(int32_t value_type, int32_t index_type, int32_t indptr_type,
+                                  const void* colptr_dev, const void* rowind_dev,
+                                  const void* data_dev, int32_t pos_type, const void* pos_dev,
+                                  const void* dC_dev, int64_t lddc, const void* B_dev, int64_t ldb,
+                                  void* dB_dev, int64_t lddb, void* dvalues_dev,
+                                  int64_t n_cols, int64_t n_dense, int64_t nnz, int64_t n_rows,
+                                  int32_t lanes_n, const fsp_csr_plan* plan, void* stream);
 
 /* Size of the static device scratch behind fsp_spmm_csr_noalloc (per GPU). */
 #define FSP_NOALLOC_SCRATCH_BYTES (16ll << 20)
