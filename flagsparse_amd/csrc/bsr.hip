@@ -451,6 +451,205 @@ __global__ __launch_bounds__(64 * WPG) void bsr_spmm_kernel(
   }
 }
 
+// The same product (same bits) for a packed B below 4 GiB.  One wave owns
+// ROWS block rows and TILES 16-column tiles and keeps one block pair of each
+// row in flight beside the pair it multiplies.  Its block columns come 64 at a
+// time, one per lane, so no pair waits for a column id before its B rows; the
+// blocks of a chunk are a buffer of their own and an absent block's B rows lie
+// past B's buffer, so both read as zeros and nothing is masked.
+//
+// What bounds it is where the B rows come from.  All waves sweep the ascending
+// block columns together and a wave that is ahead misses L2 while the others
+// hit what it brought in, so few waves with wide rows stay in step: 65536^2,
+// 40 blocks per row, N = 128, bf16 takes 56 us here (ROWS 2, TILES 8: 2048
+// waves) against 67 us with bsr_spmm_kernel's 16384 waves; four waves per block
+// row and 2 to 4 pairs in flight fetch 4.8 instead of 2.8 million lines of 128
+// bytes across the fabric and take 83-90 us.  fp8 48 -> 39 us; 20000^2, 20
+// blocks, N = 256: 25 -> 21 us; 65536^2, 20 blocks, N = 48: 37 -> 19 us.
+template <int KIND, typename BP, int TILES, int ROWS>
+__global__ __launch_bounds__(64) void bsr_spmm_sweep_kernel(
+    const BP* __restrict__ block_ptr, const int32_t* __restrict__ block_col, const void* __restrict__ block_data,
+    const float* __restrict__ block_scales, const void* __restrict__ Bp, uint32_t bp_bytes,
+    const float* __restrict__ b_absmax, int64_t n_block_rows, int64_t nbc, int64_t Npad, int64_t N,
+    float* __restrict__ C, int64_t ldc, int64_t M) {
+  using V = typename std::conditional<KIND == 0, bf16x8, f16x8>::type;
+  using AF = typename std::conditional<KIND == 2, uint64_t, V>::type;  // one lane's A (or B) fragment
+  constexpr uint32_t kFrag = sizeof(AF);   // bytes of a fragment
+  constexpr uint32_t kBlock = 32 * kFrag;  // bytes of a block
+  const int lane = threadIdx.x;
+  const int64_t nbase = static_cast<int64_t>(blockIdx.y) * (TILES * 16);
+  const int half = lane >> 5;      // which block of the pair this lane carries
+  const int r = lane & 15;         // A row / B column inside the tile
+  const int kh = (lane >> 4) & 1;  // which 8-wide half of the block's K
+  const uint32_t group = static_cast<uint32_t>(Npad) * kFrag;  // bytes of 8 packed B rows
+  const uint32_t lane_a = (r * 2 + kh) * kFrag + half * kBlock;
+  const uint32_t lane_b = kh * group + (static_cast<uint32_t>(nbase) + r) * kFrag;
+  const auto b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(Bp), 0, bp_bytes, kRawBuffer);
+
+  struct frag {
+    AF a;
+    AF b[TILES];
+  };
+  auto fetch = [](__amdgpu_buffer_rsrc_t rsrc, uint32_t off) {
+    if constexpr (KIND == 2) {
+      return __builtin_bit_cast(AF, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0));
+    } else {
+      return __builtin_bit_cast(AF, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+    }
+  };
+  struct row_state {
+    int64_t at, end;  // first block of the chunk, end of the row
+    int count;        // blocks of the chunk
+    uint32_t boff;    // lane i: where block at + i's B rows start
+    float scale;
+    frag next;
+    f32x4 acc[TILES];
+  };
+  row_state rows[ROWS];
+#pragma unroll
+  for (int w = 0; w < ROWS; ++w) {
+    const int64_t br = static_cast<int64_t>(blockIdx.x) + static_cast<int64_t>(w) * gridDim.x;
+    const bool live = br < n_block_rows;  // wave-uniform
+    rows[w].at = live ? static_cast<int64_t>(block_ptr[br]) : 0;
+    rows[w].end = live ? static_cast<int64_t>(block_ptr[br + 1]) : 0;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) rows[w].acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto load = [&](row_state& s, int pair) {  // pair < 32
+    const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(block_data) + s.at * kBlock), 0, s.count * kBlock, kRawBuffer);
+    const uint32_t b0 = __builtin_amdgcn_readlane(s.boff, 2 * pair), b1 = __builtin_amdgcn_readlane(s.boff, 2 * pair + 1);
+    const uint32_t at = (half ? b1 : b0) + lane_b;
+    s.next.a = fetch(a_rsrc, static_cast<uint32_t>(pair) * (2 * kBlock) + lane_a);
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) s.next.b[t] = fetch(b_rsrc, at + t * (16 * kFrag));
+  };
+  auto use = [&](row_state& s, int pair, const frag& f) {
+    if constexpr (KIND == 2) {
+      const int si = __builtin_bit_cast(int, s.scale);
+      const float s0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 2 * pair));
+      const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 2 * pair + 1));
+      const long a_lo = half == 0 ? static_cast<long>(f.a) : 0l;
+      const long a_hi = half == 1 ? static_cast<long>(f.a) : 0l;
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        const f32x4 p0 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a_lo, static_cast<long>(f.b[t]), z, 0, 0, 0);
+        const f32x4 p1 = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a_hi, static_cast<long>(f.b[t]), z, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s.acc[t][i] += s0 * p0[i] + s1 * p1[i];
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        if constexpr (KIND == 0) {
+          s.acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a, f.b[t], s.acc[t], 0, 0, 0);
+        } else {
+          s.acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.a, f.b[t], s.acc[t], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  for (bool more = true; more;) {  // wave-uniform: 64 blocks of every row at a time
+    int pairs = 0;
+#pragma unroll
+    for (int w = 0; w < ROWS; ++w) {
+      row_state& s = rows[w];
+      const int64_t left = s.end - s.at;
+      s.count = static_cast<int>(left < 0 ? 0 : (left < 64 ? left : 64));
+      pairs = (s.count + 1) / 2 > pairs ? (s.count + 1) / 2 : pairs;
+      s.boff = bp_bytes;  // a column outside the matrix reads as zeros too
+      s.scale = 0.f;
+      if (lane < s.count) {
+        const int64_t col = static_cast<int64_t>(block_col[s.at + lane]);
+        if (col >= 0 && col < nbc) s.boff = static_cast<uint32_t>(col) * 2u * group;
+        if constexpr (KIND == 2) s.scale = block_scales[s.at + lane];
+      }
+    }
+    if (pairs > 0) {
+#pragma unroll
+      for (int w = 0; w < ROWS; ++w) load(rows[w], 0);
+      int p = 0;
+      for (; p + 1 < pairs; ++p) {
+#pragma unroll
+        for (int w = 0; w < ROWS; ++w) {
+          const frag cur = rows[w].next;
+          load(rows[w], p + 1);
+          use(rows[w], p, cur);
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < ROWS; ++w) use(rows[w], p, rows[w].next);
+    }
+    more = false;
+#pragma unroll
+    for (int w = 0; w < ROWS; ++w) {
+      rows[w].at += 64;
+      more = more || rows[w].at < rows[w].end;
+    }
+  }
+  float bscale = 1.f;
+  if constexpr (KIND == 2) {
+    // B holding Inf / NaN (absmax not finite) makes the whole product NaN
+    const float am = b_absmax[0];
+    bscale = __builtin_isfinite(am) ? (am > 0.f ? am / kE4m3Max : 1.f) : __builtin_nanf("");
+  }
+  // D layout: lane l holds rows (l / 16) * 4 + i, column l % 16 of a tile.
+#pragma unroll
+  for (int w = 0; w < ROWS; ++w) {
+    const int64_t br = static_cast<int64_t>(blockIdx.x) + static_cast<int64_t>(w) * gridDim.x;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      const int64_t gcol = nbase + t * 16 + (lane & 15);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t grow = br * kBs + (lane >> 4) * 4 + i;
+        if (br < n_block_rows && grow < M && gcol < N) C[grow * ldc + gcol] = rows[w].acc[t][i] * bscale;
+      }
+    }
+  }
+}
+
+// Tiles per wave: the fewest fragment loads per block pair over the row of C
+// (a wave loads one A fragment and TILES B fragments; padding tiles cost as
+// much as real ones), and 2 where wider waves would be fewer than four per CU.
+static inline int bsr_sweep_tiles(int64_t n_block_rows, int64_t N) {
+  const int64_t tiles = ceil_div(N, int64_t(16));
+  int best = 8;
+  for (int t : {4, 2}) {
+    if (ceil_div(tiles, int64_t(t)) * (t + 1) < ceil_div(tiles, int64_t(best)) * (best + 1)) best = t;
+  }
+  return n_block_rows * ceil_div(tiles, int64_t(best)) < 1024 ? 2 : best;
+}
+
+// Two block rows per wave once that leaves eight waves per CU.
+template <int KIND, typename BP, int TILES>
+static int launch_bsr_sweep(const BP* bp, const int32_t* block_col, const void* block_data, const float* scales,
+                            const void* Bp, int64_t bp_bytes, const float* b_absmax, int64_t n_block_rows, int64_t nbc,
+                            int64_t Npad, int64_t N, float* C, int64_t ldc, int64_t M, hipStream_t s) {
+  const int64_t chunks = ceil_div(N, int64_t(TILES * 16));
+  if (chunks > 65535) return fail(FSP_ERR_ARG, "fsp_bsr_spmm: grid too large");
+  const auto launch = [&](auto kernel, int64_t rows) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(n_block_rows, rows)), static_cast<unsigned>(chunks));
+    hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, bp, block_col, block_data, scales, Bp,
+                       static_cast<uint32_t>(bp_bytes), b_absmax, n_block_rows, nbc, Npad, N, C, ldc, M);
+  };
+  if (n_block_rows * chunks >= 4096) {
+    launch(bsr_spmm_sweep_kernel<KIND, BP, TILES, 2>, 2);
+  } else {
+    launch(bsr_spmm_sweep_kernel<KIND, BP, TILES, 1>, 1);
+  }
+  return check_launch("bsr_spmm");
+}
+
+template <int KIND, typename BP, typename... A>
+static int launch_bsr_sweep_tiles(int tiles, A... a) {
+  if (tiles == 8) return launch_bsr_sweep<KIND, BP, 8>(a...);
+  if (tiles == 4) return launch_bsr_sweep<KIND, BP, 4>(a...);
+  return launch_bsr_sweep<KIND, BP, 2>(a...);
+}
+
 }  // namespace fsp
 
 using namespace fsp;
@@ -639,8 +838,22 @@ int fsp_bsr_spmm(int32_t value_type, int32_t block_ptr_type, const void* block_p
   if (n_block_rows > INT32_MAX || ychunks > 65535) return fail(FSP_ERR_ARG, "fsp_bsr_spmm: grid too large");
   const hipStream_t s = as_stream(stream);
   const dim3 grid(static_cast<unsigned>(n_block_rows), static_cast<unsigned>(ychunks));
+  const int64_t frag_bytes = value_type == FSP_F8E4M3 ? 8 : 16;
+  const int64_t bp_bytes = nbc * 2 * Npad * frag_bytes;
   FSP_DISPATCH_INDEX(block_ptr_type, BP, {
     const BP* bp = static_cast<const BP*>(block_ptr_dev);
+    // 32-bit offsets into B, with room for the offsets of absent blocks
+    if (bp_bytes + 2 * Npad * frag_bytes < (int64_t(1) << 32)) {
+      const auto sweep = [&](auto kind) {
+        return launch_bsr_sweep_tiles<decltype(kind)::value, BP>(
+            bsr_sweep_tiles(n_block_rows, N), bp, block_col_dev, block_data_dev, block_scales_dev, Bp_dev, bp_bytes,
+            b_absmax_dev, n_block_rows, nbc, Npad, N, C_dev, ldc, M, s);
+      };
+      if (value_type == FSP_BF16) return sweep(std::integral_constant<int, 0>{});
+      if (value_type == FSP_F16) return sweep(std::integral_constant<int, 1>{});
+      if (value_type == FSP_F8E4M3) return sweep(std::integral_constant<int, 2>{});
+      return fail(FSP_ERR_DTYPE, "fsp_bsr_spmm: value type %d has no MFMA path", (int)value_type);
+    }
     if (value_type == FSP_BF16) {
       hipLaunchKernelGGL((bsr_spmm_kernel<0, BP, 4>), grid, dim3(64 * 4), 0, s, bp, block_col_dev, block_data_dev,
                          nullptr, Bp_dev, nullptr, nbc, Npad, N, C_dev, ldc, M);

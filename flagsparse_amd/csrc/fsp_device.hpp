@@ -173,6 +173,9 @@ __device__ __forceinline__ const P& elem(const P* base, typename addr<OFF32>::of
   return *addr<OFF32>::at(base, i * static_cast<typename addr<OFF32>::off_t>(sizeof(P)));
 }
 
+// Third word of a raw buffer descriptor (32-bit elements, no swizzle).
+constexpr int kRawBuffer = 0x00020000;
+
 // ------------------------------------------------------------ index helpers
 template <typename I> __device__ __forceinline__ int64_t ld_idx(const I* p, int64_t i) {
   return static_cast<int64_t>(p[i]);

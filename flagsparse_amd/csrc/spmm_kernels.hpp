@@ -290,9 +290,6 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
   }
 }
 
-// Third word of a raw buffer descriptor (32-bit elements, no swizzle).
-constexpr int kRawBuffer = 0x00020000;
-
 // n elements of E (below 4 GiB) as a buffer: element kAbsent reads as zero and
 // touches no memory.
 constexpr uint32_t kAbsent = ~0u;
