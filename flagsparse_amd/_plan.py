@@ -236,10 +236,12 @@ _N_STATS = 6  # figures ahead of the bin offsets in fsp_csr_build_plan's meta
 _KEEP_BYTES = 1 << 20
 
 
-def _build(indptr, indices, n_rows, nnz, config):
+def _build(indptr, indices, n_rows, nnz, config, meanwhile=None):
     """fsp_csr_build_plan and the one host readback: (figures, plan arrays).
     The plan arrays are None without `config`; they are usable only if the
-    figures describe a valid CSR of at most nnz nonzeros."""
+    figures describe a valid CSR of at most nnz nonzeros.  meanwhile() is
+    called between the copy of the figures and the wait for it: what it
+    launches runs while the host waits and goes on."""
     device = indptr.device
     lib = _lib.load()
     n_bins = len(config.uppers) + 1 if config is not None else 0  # regular bins + the long bin
@@ -269,7 +271,15 @@ def _build(indptr, indices, n_rows, nnz, config):
         ),
         "fsp_csr_build_plan",
     )
-    host = buf[:n_meta].tolist()  # the one host sync
+    if meanwhile is None:
+        host = buf[:n_meta].tolist()  # the one host sync
+    else:
+        stream = torch.cuda.current_stream(device)
+        figures = buf[:n_meta].to("cpu", non_blocking=True)
+        copied = stream.record_event()
+        meanwhile()
+        copied.synchronize()  # the one host sync, behind the copy only
+        host = figures.tolist()
     if not n_bins:
         return host, None
     off, n_seg = host[_N_STATS:-1], host[-1]
@@ -301,14 +311,14 @@ def build_plan(indptr, n_rows, config, nnz=None):
     return _finish_plan(indptr, n_rows, config, arrays, _row_len_if_constant(n_rows, first, last, max_len), first)
 
 
-def inspect_csr(indptr, indices, n_rows, nnz, config=None):
+def inspect_csr(indptr, indices, n_rows, nnz, config=None, meanwhile=None):
     """Validation figures of a CSR and, with `config`, its row-bin plan, for
     ONE host readback.  Returns (stats, plan): stats has indptr_first,
     indptr_last, n_decreasing, min_col, max_col (None without nonzeros) and
     max_row; plan is None without `config` or when the row pointer is not a
     valid CSR (the caller raises on the stats first)."""
     n_rows, nnz = int(n_rows), int(nnz)
-    host, arrays = _build(indptr, indices, n_rows, nnz, config)
+    host, arrays = _build(indptr, indices, n_rows, nnz, config, meanwhile)
     stats = {
         "indptr_first": host[0],
         "indptr_last": host[1],

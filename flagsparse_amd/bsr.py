@@ -21,6 +21,7 @@ import torch
 from . import _lib, _plan
 
 BLOCK_DIM = 16
+_DENSE_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
 _BSR_KERNEL_DTYPES = (torch.bfloat16, torch.float16, torch.uint8)  # uint8 = FP8 e4m3 codes
 
 
@@ -28,12 +29,13 @@ def _padded_cols(n):
     return -(-int(n) // 128) * 128
 
 
-def _validate_bsr(data, indices, indptr, shape, block_dim):
+def _validate_bsr(data, indices, indptr, shape, block_dim, meanwhile=None):
     """Validation contract of the reference's _prepare_spmv_bsr_matrix
     (spmv_bsr.py:448-490): same checks, same messages, for block_dim 16.
     Returns (data, block columns as int32, indptr, n_rows, n_cols,
     n_block_rows, n_block_cols); int64 block columns are narrowed to int32
-    (after the range check) because the MFMA kernel reads int32."""
+    (after the range check) because the MFMA kernel reads int32.
+    meanwhile(): see _plan.inspect_csr."""
     if not all(torch.is_tensor(t) for t in (data, indices, indptr)):
         raise TypeError("data, indices, indptr must all be torch.Tensor")
     if data.ndim != 3:
@@ -69,7 +71,7 @@ def _validate_bsr(data, indices, indptr, shape, block_dim):
     indptr = indptr.contiguous()
     # every check from one device inspection and one host readback
     nnzb = int(indices.numel())
-    stats, _ = _plan.inspect_csr(indptr, indices, n_block_rows, nnzb)
+    stats, _ = _plan.inspect_csr(indptr, indices, n_block_rows, nnzb, meanwhile=meanwhile)
     if stats["indptr_first"] != 0:
         raise ValueError("indptr must start at zero")
     if stats["indptr_last"] != data.shape[0]:
@@ -187,7 +189,18 @@ def flagsparse_spmm_bsr(data, indices, indptr, B, shape, block_dim=BLOCK_DIM, sc
     or f16); for bf16/f16 blocks B is converted to the block dtype, for FP8 it
     is quantised with one absmax scale per tensor.  Accumulation is float32.
     """
-    data, indices, indptr, n_rows, n_cols, n_block_rows, _ = _validate_bsr(data, indices, indptr, shape, block_dim)
+    packed = []
+
+    def pack():
+        # B is packed while the host waits for the figures of the matrix, if it
+        # is an operand that the checks below will accept (an error of the
+        # matrix still comes first and drops the packed B)
+        if (torch.is_tensor(B) and B.ndim == 2 and B.shape[0] == int(shape[1]) and B.is_cuda
+                and B.device == data.device and B.dtype in _DENSE_DTYPES and int(shape[0]) and B.numel()):
+            packed.append(pack_dense_operand(B, data.dtype))
+
+    data, indices, indptr, n_rows, n_cols, n_block_rows, _ = _validate_bsr(data, indices, indptr, shape, block_dim,
+                                                                           pack)
     fp8 = data.dtype == torch.uint8
     if fp8 and (scales is None or scales.numel() != data.shape[0] or scales.dtype != torch.float32
                 or not scales.is_cuda or scales.device != data.device):
@@ -200,7 +213,7 @@ def flagsparse_spmm_bsr(data, indices, indptr, B, shape, block_dim=BLOCK_DIM, sc
         raise ValueError(f"B.shape[0] must be n_cols={n_cols}, got {B.shape[0]}")
     if not B.is_cuda or B.device != data.device:
         raise ValueError("B must be a CUDA tensor on the same device as the sparse matrix")
-    if B.dtype not in (torch.float32, torch.bfloat16, torch.float16):
+    if B.dtype not in _DENSE_DTYPES:
         raise TypeError("B dtype must be float32, bfloat16 or float16")
     N = int(B.shape[1])
     device = data.device
@@ -211,7 +224,7 @@ def flagsparse_spmm_bsr(data, indices, indptr, B, shape, block_dim=BLOCK_DIM, sc
         raise ValueError("out must be a contiguous float32 tensor of shape (n_rows, N) on the matrix's device")
     if n_rows == 0 or N == 0:
         return out
-    Bp, absmax = pack_dense_operand(B, torch.uint8 if fp8 else data.dtype)
+    Bp, absmax = packed[0] if packed else pack_dense_operand(B, data.dtype)
     scales = None if scales is None else scales.contiguous()
     vcode = _lib.FSP_F8E4M3 if fp8 else _lib.value_code(data.dtype)
     _lib.check(
