@@ -202,7 +202,7 @@ class CsrHandle:
         y = out if out is not None else torch.empty(n_out, dtype=data.dtype, device=x.device)
         if n_out == 0:
             return y
-        cfg = config or _plan.spmv_config()
+        cfg = config or (_plan.spmv_config() if variant else _plan.spmv_wide_config())
         if transpose:
             colptr, rowind, perm = self.csc()
             plan = self.csc_plan(cfg)

@@ -12,7 +12,8 @@ costs no host sync.
 Bin layouts per kernel family (``unroll`` = nonzeros per lane per trip):
 
 * SpMV: lanes per row L in {4, 8, 16, 32, 64}; a row of length n goes to the
-  smallest L with n <= L * unroll, L = 64 up to ``long_threshold``.
+  smallest L with n <= L * unroll, L = 64 up to ``long_threshold`` (untuned
+  pipelined loop: up to 1024, then a workgroup's 256 lanes).
 * SpMM / SDDMM with G lanes along the dense dimension: nonzero slots per row
   S in {1, 2, ..., 64 / G}; smallest S with n <= S * unroll * slot_scale,
   S = 64 / G up to ``long_threshold``.  SDDMM uses half the lanes of a full
@@ -35,6 +36,8 @@ from . import _lib
 SPMV_UNROLL = 4
 SPMV_LONG_THRESHOLD = 4096
 SPMV_SEG_LEN = 4096
+SPMV_WIDE_ROW = 1024  # the pipelined loop's rows above this take a workgroup
+SPMV_WIDE_LANES = 256
 SPMM_UNROLL = 4
 SPMM_LONG_THRESHOLD = 256
 SPMM_SEG_LEN = 256
@@ -85,6 +88,23 @@ def spmv_config(unroll=SPMV_UNROLL, long_threshold=SPMV_LONG_THRESHOLD, seg_len=
     lanes = (4, 8, 16, 32, 64)
     uppers = [min(l * unroll, long_threshold) for l in lanes[:-1]] + [long_threshold]
     return _dedupe(lanes, uppers, seg_len, unroll)
+
+
+@lru_cache(maxsize=1)
+def spmv_wide_config():
+    """Bins of the software-pipelined loop without tuning: as spmv_config, but
+    rows of more than 1024 nonzeros and the segments of long ones take a
+    workgroup each.  f32, 100000 rows of 10 on average: power-law up to 4096 /
+    with 20 rows of 9000, microseconds: one wave a row 15.6 / 20.4; a workgroup
+    above 256: 11.2, above 512: 10.7 / 12.6, above 1024: 10.5 / 12.6, above 2048:
+    11.1."""
+    base = spmv_config(long_threshold=SPMV_WIDE_ROW)
+    return PlanConfig(base.lanes + (SPMV_WIDE_LANES,), base.uppers + (SPMV_LONG_THRESHOLD,), SPMV_SEG_LEN, SPMV_UNROLL)
+
+
+def spmv_plan_config(x_len, elem_bytes, nnz):
+    """Bins for the loop that spmv_default_variant picks."""
+    return spmv_config() if spmv_default_variant(x_len, elem_bytes, nnz) else spmv_wide_config()
 
 
 @lru_cache(maxsize=1024)

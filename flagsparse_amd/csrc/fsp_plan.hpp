@@ -180,13 +180,14 @@ static int64_t build_launch_table(const fsp_csr_plan* plan, int seg_lanes_log2, 
   return blocks;
 }
 
-static inline int check_plan(const fsp_csr_plan* plan, int64_t n_rows) {
+// max_lanes: most lanes that one row may take (64; the SpMV also a workgroup).
+static inline int check_plan(const fsp_csr_plan* plan, int64_t n_rows, int max_lanes = 64) {
   if (plan == nullptr) return fail(FSP_ERR_ARG, "plan is NULL");
   if (plan->n_bins < 0 || plan->n_bins > FSP_MAX_BINS) return fail(FSP_ERR_ARG, "plan: bad n_bins %d", plan->n_bins);
   int64_t total = 0;
   for (int i = 0; i < plan->n_bins; ++i) {
     const fsp_bin& b = plan->bins[i];
-    if (b.count < 0 || b.lanes < 1 || b.lanes > 64 || !is_pow2(b.lanes)) {
+    if (b.count < 0 || b.lanes < 1 || b.lanes > max_lanes || !is_pow2(b.lanes)) {
       return fail(FSP_ERR_ARG, "plan: bin %d has count %lld lanes %d", i, (long long)b.count, b.lanes);
     }
     if (b.rows == nullptr && b.count > n_rows) return fail(FSP_ERR_ARG, "plan: identity bin larger than n_rows");

@@ -16,7 +16,7 @@ extern "C" int fsp_spmv_csr(int32_t value_type, int32_t index_type, int32_t indp
                             int32_t perm_type, const void* perm_dev, const void* x_dev, void* y_dev,
                             int64_t n_rows, int64_t nnz, int64_t x_len, const fsp_csr_plan* plan, void* stream) {
   if (n_rows < 0 || nnz < 0 || x_len < 0) return fail(FSP_ERR_ARG, "fsp_spmv_csr: negative n_rows, nnz or x_len");
-  int st = check_plan(plan, n_rows);
+  int st = check_plan(plan, n_rows, kWideLanes);
   if (st) return st;
   if (n_rows == 0) return FSP_OK;
   if (indptr_dev == nullptr || y_dev == nullptr) return fail(FSP_ERR_ARG, "fsp_spmv_csr: NULL indptr or y");

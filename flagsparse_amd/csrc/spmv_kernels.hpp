@@ -2,8 +2,8 @@
 //
 // Rows are binned by length; a bin with lanes L puts 64/L rows on one wave and
 // splits each row's nonzeros over L lanes, then a DPP group sum.  Rows longer
-// than the last bin are cut into segments; one wave reduces each segment into
-// a partial and a second pass adds a row's partials in segment order (no
+// than the last bin are cut into segments; one wave (a workgroup, if the plan
+// has a bin of workgroup rows) reduces each segment into a partial and a second pass adds a row's partials in segment order (no
 // atomics: the result is deterministic for a plan).  One fused launch runs
 // every bin and the segments with the loop plan.variant selects:
 //   0  spmv_bins_kernel: lane l takes nonzeros l, l+L, ..., UNROLL loads in
@@ -16,8 +16,9 @@
 //      x in LDS; a plan whose rows all have one length (plan.row_len) runs
 //      its own instantiation that computes the row bounds and, when a row
 //      fits one trip, software-pipelines the row tiles.
-// Variants 0-3 are bitwise equal, and so are variant 4's two forms.  spmv_parts_kernel (fsp_spmv_csr_parts)
-// runs row-range parts, each with its own column window of x in LDS (the
+// Variants 0-3 are bitwise equal on plans without a bin of workgroup rows, and
+// so are variant 4's two forms.  spmv_parts_kernel (fsp_spmv_csr_parts) runs
+// row-range parts, each with its own column window of x in LDS (the
 // batched SpMV).
 #pragma once
 
@@ -163,6 +164,14 @@ __device__ __forceinline__ const T* stage_x(const T* __restrict__ x, int64_t x_l
   }
 }
 
+// A plan bin of kWideLanes lanes gives each of its rows a workgroup.  One wave
+// needs 16 trips, a memory round trip each, for a row of 4096 nonzeros, and the
+// launch waits for its last row: the bound is that chain, not the traffic.
+// With a workgroup above 1024 nonzeros, power-law rows of up to 4096, f32:
+// 100000 rows of 10 on average 15.6 -> 10.5 us, 50000 of 24 17.8 -> 12.6,
+// 262144 of 24 37.1 -> 35.1 (its 6.3 M gathers of x take 29 us by themselves).
+constexpr int kWideLanes = FSP_WG_THREADS;
+
 template <typename T, typename IT, typename PT, typename QT, int UNROLL, bool PERM, int WAVES, bool LDSX>
 __global__ __launch_bounds__(64 * WAVES) void spmv_bins_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const T* __restrict__ data,
@@ -177,10 +186,14 @@ __global__ __launch_bounds__(64 * WAVES) void spmv_bins_kernel(
   const int L = 1 << ll;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int sub = lane >> ll;
-  const int l = lane & (L - 1);
-  const int64_t per_wave = 64 >> ll;
-  const int64_t per_block = per_wave * WAVES;
+  // kWideLanes: all of the workgroup's waves on one row at a time (the table
+  // holds at most 64 lanes for workgroups of other sizes)
+  constexpr bool kWide = !LDSX && WAVES * 64 == kWideLanes;
+  const bool wide = kWide && L == kWideLanes;  // uniform over the workgroup
+  const int sub = wide ? 0 : lane >> ll;
+  const int l = wide ? static_cast<int>(threadIdx.x) : lane & (L - 1);
+  const int64_t per_wave = wide ? 0 : 64 >> ll;
+  const int64_t per_block = wide ? 1 : per_wave * WAVES;
   const tile_range tr = bin_tiles(lb, per_block);
   const int64_t rr_step = tr.step * per_block;
   const int64_t last_item = lb.count - 1;  // bins in the table are non-empty
@@ -246,7 +259,16 @@ __global__ __launch_bounds__(64 * WAVES) void spmv_bins_kernel(
       }
     }
     if (!prefetched && has_next) trip(beg_n + l, end_n, c, a);
-    acc = group_sum(acc, L);
+    acc = group_sum(acc, L < 64 ? L : 64);
+    if constexpr (kWide) {
+      __shared__ A s_wave[WAVES];
+      if (wide) {
+        if (lane == 0) s_wave[wave] = acc;
+        __syncthreads();
+        acc = (s_wave[0] + s_wave[1]) + (s_wave[2] + s_wave[3]);
+        __syncthreads();  // before the next row's sums
+      }
+    }
     if (active && l == 0) {
       if (lb.is_segment) {
         partials[out] = acc;
@@ -886,9 +908,15 @@ static int launch_spmv(const void* indptr, const void* indices, const void* data
     lplan.max_blocks = 2 * static_cast<int64_t>(cus > 0 ? cus : 256);
   }
   const int64_t waves = ldsx ? kLdsxWaves : FSP_WAVES;
+  // a plan that gives long rows a workgroup cuts its segments for one, too
+  const int max_ll = plan->variant == 0 ? ilog2(kWideLanes) : 6;
+  int seg_ll = 6;
+  for (int i = 0; i < plan->n_bins; ++i) {
+    if (plan->bins[i].lanes == kWideLanes) seg_ll = max_ll;
+  }
   const int64_t blocks = build_launch_table(
-      &lplan, /*seg_lanes_log2=*/6, /*max_lanes_log2=*/6,
-      [waves](int ll, int) { return waves * (int64_t(64) >> ll); }, &tab);
+      &lplan, seg_ll, max_ll,
+      [waves](int ll, int) { return ll > 6 ? int64_t(1) : waves * (int64_t(64) >> ll); }, &tab);
   if (plan->n_segments > 0 &&
       (plan->partials_dev == nullptr || plan->partials_bytes < plan->n_segments * (int64_t)sizeof(A))) {
     return fail(FSP_ERR_WORKSPACE, "fsp_spmv_csr: partials need %lld bytes",

@@ -119,8 +119,9 @@ class PreparedCsrSpmv:
     def plan(self, config=None):
         """The row-bin plan of this matrix (built on first use, then cached)."""
         if self._plan is None or (config is not None and self._plan.config != config):
-            self._plan = _plan.build_plan(self.kernel_indptr, self.n_rows, config or _plan.spmv_config(),
-                                          self.kernel_indices.numel())
+            nnz = self.kernel_indices.numel()
+            config = config or _plan.spmv_plan_config(self.n_cols, self.data.element_size(), nnz)
+            self._plan = _plan.build_plan(self.kernel_indptr, self.n_rows, config, nnz)
         return self._plan
 
 
@@ -148,8 +149,8 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy
     return _inspect_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy)[0]
 
 
-def _inspect_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy="auto", plan_config=None):
-    """_prepare_spmv_csr_matrix plus, with `plan_config`, the row-bin plan,
+def _inspect_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy="auto", with_plan=False):
+    """_prepare_spmv_csr_matrix plus, if asked for, the row-bin plan,
     from one device inspection and ONE host readback (the reference makes a
     host sync per check).  Returns (validated tuple, plan or None)."""
     _normalize_spmv_index_fallback_policy(index_fallback_policy)
@@ -177,6 +178,7 @@ def _inspect_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy
     indices = indices.contiguous()
     indptr = indptr.contiguous()
     nnz = data.numel()
+    plan_config = _plan.spmv_plan_config(n_cols, data.element_size(), nnz) if with_plan else None
     stats, plan = _plan.inspect_csr(indptr, indices, n_rows, nnz, plan_config)
     if stats["indptr_first"] != 0:
         raise ValueError("indptr must start at zero")
@@ -233,7 +235,7 @@ def prepare_spmv_csr(
             data = data.conj().resolve_conj()
         data, indices, indptr, shape = _transpose_csr_for_spmv(data, indices, indptr, shape)
     (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths, max_row_nnz), plan = _inspect_spmv_csr_matrix(
-        data, indices, indptr, shape, index_fallback_policy=index_fallback_policy, plan_config=_plan.spmv_config()
+        data, indices, indptr, shape, index_fallback_policy=index_fallback_policy, with_plan=True
     )
     # block_nnz / max_segments keep the caller's launch hints in the prepared
     # object's public slots; the HIP kernel takes its split from the plan

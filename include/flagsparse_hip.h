@@ -47,7 +47,9 @@ typedef enum fsp_status {
 } fsp_status;
 
 /* One row-length bin of a CSR work plan.  `lanes` is the number of lanes that
- * cooperate on one row: SpMV splits a row's nonzeros over `lanes` lanes; SpMM
+ * cooperate on one row: SpMV splits a row's nonzeros over `lanes` lanes (1..64,
+ * or 256 = the workgroup, which only variant 0 takes in full, as it then does
+ * for the segments; the others run such bins with 64); SpMM
  * and SDDMM split them over `lanes` nonzero slots (each slot spans the lanes
  * that cover the dense dimension). */
 typedef struct fsp_bin {
