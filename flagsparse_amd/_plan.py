@@ -189,6 +189,17 @@ class CsrPlan:
     indptr_base: int = 0  # indptr[0] when row_len > 0
     _structs: dict = field(default_factory=dict, init=False, repr=False, compare=False)
 
+    # The structs hold the addresses of this plan's own tensors: a copy, a pickle
+    # or a plan that was saved before there were any starts without them.
+    def __getstate__(self):
+        state = dict(self.__dict__)
+        state.pop("_structs", None)
+        return state
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._structs = {}
+
     @property
     def bin_sizes(self):
         return list(self.bin_counts) + [self.n_long_rows]
