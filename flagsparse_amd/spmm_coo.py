@@ -172,7 +172,7 @@ class _CanonicalCoo:
         """C = op(A) B in the requested layout (row-major kernel): B and C in
         the input dtype, products and sums in the values' compute dtype."""
         n_rows = self.shape[0]
-        B_row = B.contiguous()
+        B_row = B.contiguous().resolve_neg()
         # the kernel writes a contiguous `out` itself unless it is B's own
         # memory; an `out` in the autograd graph gets copy_'s checks
         direct = (out if out is not None and out.is_contiguous() and not out.requires_grad

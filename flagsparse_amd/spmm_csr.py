@@ -338,7 +338,7 @@ class PreparedCsrSpmmOpt:
     def _describe(self, plan):
         """Fill the reference's bucket / split fields from a HIP plan (once
         per plan: a launch of the same plan has nothing to add)."""
-        if self._described is plan:
+        if getattr(self, "_described", None) is plan:  # absent in an object saved without it
             return
         self._described = plan
         self.row_buckets = [
