@@ -157,30 +157,33 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void fill_i64_kernel(int64_t* __res
 
 template <int BYTES> struct blob { alignas(BYTES < 16 ? BYTES : 16) unsigned char b[BYTES]; };
 
-// out[q] = in[perm[q]].  Each thread moves kGatherItems consecutive elements:
-// its permutation entries come as whole vectors, its reads of `in` are all in
+// out[q] = in[perm[q]].  Each thread moves ITEMS consecutive elements: its
+// permutation entries come as whole vectors, its reads of `in` are all in
 // flight together and its results leave as vectors.  The reads are what
 // bounds it: each is a cache line of its own, 2.5-2.8 clocks per line and CU
-// from L2 (2.8 M values of 2 bytes: 21.8 us
-// with one element per thread, 18.0 us with four, 19.4 with eight).
+// from L2 (2.8 M values of 2 bytes: 21.8 us with one element per thread, 18.0
+// us with four, 19.4 with eight).  Values well beyond the L2s come across the
+// fabric, which more reads in flight slow down: 11 MB 30.0 us with one element
+// per thread and 30.2 with four, 12.5 MB 50.3 and 51.2, 25 MB 66.9 and 68.8.
 constexpr int kGatherItems = 4;
-template <int BYTES, typename QT>
+constexpr int64_t kGatherWideBytes = int64_t(8) << 20;  // four up to here, one beyond
+template <int BYTES, typename QT, int ITEMS>
 __global__ __launch_bounds__(FSP_WG_THREADS) void gather_kernel(
     const QT* __restrict__ perm, const blob<BYTES>* __restrict__ in, blob<BYTES>* __restrict__ out,
     int64_t n) {
-  struct perms { QT q[kGatherItems]; };
-  struct items { blob<BYTES> v[kGatherItems]; };
-  const int64_t whole = n / kGatherItems;
+  struct perms { QT q[ITEMS]; };
+  struct items { blob<BYTES> v[ITEMS]; };
+  const int64_t whole = n / ITEMS;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * FSP_WG_THREADS;
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * FSP_WG_THREADS + threadIdx.x;
   for (int64_t i = tid; i < whole; i += stride) {
-    const perms p = *reinterpret_cast<const perms*>(perm + i * kGatherItems);
+    const perms p = *reinterpret_cast<const perms*>(perm + i * ITEMS);
     items o;
 #pragma unroll
-    for (int k = 0; k < kGatherItems; ++k) o.v[k] = in[static_cast<int64_t>(p.q[k])];
-    *reinterpret_cast<items*>(out + i * kGatherItems) = o;
+    for (int k = 0; k < ITEMS; ++k) o.v[k] = in[static_cast<int64_t>(p.q[k])];
+    *reinterpret_cast<items*>(out + i * ITEMS) = o;
   }
-  const int64_t q = whole * kGatherItems + tid;
+  const int64_t q = whole * ITEMS + tid;
   if (q < n) out[q] = in[static_cast<int64_t>(perm[q])];
 }
 
@@ -304,18 +307,30 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void csr_stats_kernel(const PT* __r
   }
 }
 
-template <typename QT>
-static int launch_gather(int32_t elem_bytes, const QT* perm, const void* in, void* out, int64_t n, hipStream_t s) {
-  const dim3 grid(grid_for(ceil_div(n, int64_t(kGatherItems)))), block(FSP_WG_THREADS);
-  switch (elem_bytes) {
-    case 1: hipLaunchKernelGGL((gather_kernel<1, QT>), grid, block, 0, s, perm, static_cast<const blob<1>*>(in), static_cast<blob<1>*>(out), n); break;
-    case 2: hipLaunchKernelGGL((gather_kernel<2, QT>), grid, block, 0, s, perm, static_cast<const blob<2>*>(in), static_cast<blob<2>*>(out), n); break;
-    case 4: hipLaunchKernelGGL((gather_kernel<4, QT>), grid, block, 0, s, perm, static_cast<const blob<4>*>(in), static_cast<blob<4>*>(out), n); break;
-    case 8: hipLaunchKernelGGL((gather_kernel<8, QT>), grid, block, 0, s, perm, static_cast<const blob<8>*>(in), static_cast<blob<8>*>(out), n); break;
-    case 16: hipLaunchKernelGGL((gather_kernel<16, QT>), grid, block, 0, s, perm, static_cast<const blob<16>*>(in), static_cast<blob<16>*>(out), n); break;
-    default: return fail(FSP_ERR_ARG, "fsp_gather: unsupported element size %d", (int)elem_bytes);
+template <int BYTES, typename QT>
+static int launch_gather_blob(const QT* perm, const void* in, void* out, int64_t n, hipStream_t s) {
+  const auto launch = [&](auto kernel, int64_t items) {
+    hipLaunchKernelGGL(kernel, dim3(grid_for(ceil_div(n, items))), dim3(FSP_WG_THREADS), 0, s, perm,
+                       static_cast<const blob<BYTES>*>(in), static_cast<blob<BYTES>*>(out), n);
+  };
+  if (n * BYTES > kGatherWideBytes) {
+    launch(gather_kernel<BYTES, QT, 1>, 1);
+  } else {
+    launch(gather_kernel<BYTES, QT, kGatherItems>, kGatherItems);
   }
   return check_launch("gather");
+}
+
+template <typename QT>
+static int launch_gather(int32_t elem_bytes, const QT* perm, const void* in, void* out, int64_t n, hipStream_t s) {
+  switch (elem_bytes) {
+    case 1: return launch_gather_blob<1>(perm, in, out, n, s);
+    case 2: return launch_gather_blob<2>(perm, in, out, n, s);
+    case 4: return launch_gather_blob<4>(perm, in, out, n, s);
+    case 8: return launch_gather_blob<8>(perm, in, out, n, s);
+    case 16: return launch_gather_blob<16>(perm, in, out, n, s);
+    default: return fail(FSP_ERR_ARG, "fsp_gather: unsupported element size %d", (int)elem_bytes);
+  }
 }
 
 }  // namespace fsp

@@ -37,7 +37,7 @@ def test_permuted_and_gathered_values_agree(device, dtype, n, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.float64, torch.complex128])
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 70001])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 70001, (8 << 20) // 8, (8 << 20) // 8 + 1])
 def test_gather_remainders(device, dtype, n):
     x = torch.tensor(np.random.default_rng(n).integers(0, 100, n + 1), device=device).to(dtype)[1:]  # off alignment
     for perm_dtype in (torch.int32, torch.int64):
