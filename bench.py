@@ -7,7 +7,7 @@ in HBM): C = A B, A 262144 x 262144 CSR with power-law row lengths (exponent
 
 value = algorithmic bytes / time per step (GB/s), where algorithmic bytes =
 nnz*(4+4) + (M+1)*4 + K*N*4 + M*N*4 (A streamed once, B read once, C written
-once).  The roofline object prices the dominant kernel (spmm_bins_kernel)
+once).  The roofline object prices the dominant kernel (spmm_slots_kernel)
 against the 8 TB/s HBM peak with its duration from HIP events on the stream
 the kernels run on.  The same line also carries the bf16-vs-fp32 fwd+bwd
 speedup of the differentiable SpMM (200000-node power-law graph, N=128) and
@@ -780,7 +780,7 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(),
-            "kernel": "spmm_bins_kernel (+ spmm_long_reduce_kernel inside the event window)",
+            "kernel": "spmm_slots_kernel (+ spmm_long_reduce_kernel inside the event window)",
             "kernel_ms": round(kern_ms, 5),
         },
         "plan": r["plan"],

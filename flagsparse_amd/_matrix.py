@@ -3,11 +3,11 @@
 A ``CsrHandle`` owns (references to) indptr / indices and caches, per kernel
 configuration, the row-bin plans of the CSR and -- on first transposed use --
 the stable CSC permutation (colptr, rowind, perm) with its own plans.  Only
-the index structure is cached: a transposed SpMM gathers the values into CSC
-order on every call (``fsp_gather`` into a buffer of the caching allocator)
-and runs the plain kernel over the CSC, so a handle stays valid while the
-values change (training).  The transposed SpMV reads them through ``perm``
-(data[perm[q]]) inside its kernel.  All launches go through the C ABI of
+the index structure is cached, so a handle stays valid while the values change
+(training): a transposed SpMM reads a small value array through ``perm``
+(data[perm[q]]) inside its kernel and gathers a larger one into CSC order on
+every call (``fsp_gather`` into a buffer of the caching allocator, see
+_permuted_in_kernel).  The transposed SpMV always reads through ``perm``.  All launches go through the C ABI of
 libflagsparse_hip.so.
 """
 

@@ -3,8 +3,8 @@
 C = A B with A given by (values, indices, indptr, shape).  Backward:
 
 * dB = A^T dC: the transposed SpMM kernel over the handle's cached stable CSC
-  permutation (values gathered into CSC order per call; no transposed copy
-  of A's indices, no atomics);
+  permutation (values of the call, read through the permutation or gathered
+  into CSC order; no transposed copy of A's indices, no atomics);
 * dA.values = SDDMM(dC, B) on A's pattern: dvalues[p] = <dC[row p], B[col p]>.
 
 When both are needed they come from one kernel pass over the CSC
