@@ -41,9 +41,10 @@ def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes):
     68, where each of those reads is another 128 bytes across the fabric."""
     elem = data.element_size()
     dense = rows * ld * elem
+    paced = (24 if lanes >= 32 and n_dense * elem * 8 >= 16 * 7 * lanes else 64) << 20
     return (perm.numel() * elem <= _PERMUTED_BYTES and lanes >= 4 and n_dense >= 16 // elem
             and perm.dtype == torch.int32 and dense + ld * elem < 1 << 32 and n_out * n_dense * elem < 1 << 32
-            and (lanes < 16 or dense < 64 << 20))
+            and (lanes < 16 or dense < paced))
 
 
 class CsrHandle:
@@ -177,7 +178,9 @@ class CsrHandle:
         colptr, rowind, perm = self.csc()
         plan = self.csc_plan(cfg)
         name = "fsp_spmm_csr_trans_sddmm"
-        if self.nnz and not _permuted_in_kernel(data, perm, int(dC.stride(0)), self.n_rows, self.n_cols, n_dense, G):
+        # (this kernel is not paced at the wide groups' lower size)
+        if self.nnz and not _permuted_in_kernel(data, perm, int(dC.stride(0)), self.n_rows, self.n_cols, n_dense,
+                                                min(G, 16)):
             data = gather_values(data, perm)
         elif self.nnz:
             name = "fsp_spmm_csr_trans_sddmm_perm"

@@ -300,7 +300,14 @@ constexpr uint32_t kAbsent = ~0u;
 // five workgroups per CU, 228 us with spmm_slots_kernel; N = 160 558 against
 // 543 us).  Below that size the faster issue wins (200000-node graph, bf16
 // N = 128: 86 against 89 us; 50000 nodes, f32 N = 64: 24 against 26 us).
+// Rows of 512 bytes or more that use nearly every lane of their group are paced
+// from 24 MiB on: a wave load brings 1 KiB there and issuing is no bound (slots
+// against bins: 100000^2, f64 N = 64 166 / 173 us, f32 N = 128 171 / 174.5; 50000^2,
+// 25 MB of B, f32 N = 128 80.8 / 83.8, bf16 N = 256 84.8 / 87.5; 10 MB, f64 N = 64
+// 37.8 / 32.8).  With fewer lanes in use the faster issue wins (f64 N = 75, 42 MB
+// of B, 38 of 64 lanes: 290 / 242).
 constexpr int64_t kPacedBytes = int64_t(64) << 20;
+constexpr int64_t kPacedWideBytes = int64_t(24) << 20;
 template <typename E>
 struct buffer {
   __amdgpu_buffer_rsrc_t rsrc;
@@ -318,9 +325,11 @@ struct buffer {
   }
 };
 
-// Workgroups per CU (waves per SIMD) the registers must allow.
-template <int UNROLL, bool SDD>
-constexpr int kMinBlocks = SDD ? 5 : (UNROLL > 4 ? 6 : 8);
+// Workgroups per CU (waves per SIMD) the registers must allow: the most that
+// spills nothing (eight vectors of 16-bit elements need 95 registers; held to 80
+// they spill, and 200000 nodes, N = 128, unroll 8 took 116 us, 87 without).
+template <int UNROLL, bool SDD, int ELEM>
+constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : 8) : (SDD ? 4 : (ELEM == 2 ? 5 : 6));
 
 // The same layout and summation order as spmm_slots_kernel (bitwise equal),
 // with the id and value of a nonzero loaded once per quad (LANES 4) or row of
@@ -338,7 +347,7 @@ constexpr int kMinBlocks = SDD ? 5 : (UNROLL > 4 ? 6 : 8);
 // 200000-node graph, bf16 N = 128: 89 -> 86 us, its backward 144 -> 141 us.
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool PERM,
           bool SDD, bool TAIL>
-__global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD>)) void spmm_bins_kernel(
+__global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cast<int>(sizeof(T))>)) void spmm_bins_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
     const T* __restrict__ B, int64_t ldb, uint32_t b_bytes, T* __restrict__ C, int64_t ldc, int64_t n_dense, uint32_t nnz,
     int g_log2, typename acc_of<TV>::type* __restrict__ partials, launch_table tab, sdd_args<T, QT> sd) {
@@ -625,7 +634,8 @@ static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_
       }
     };
     // (b_bytes + a row stays below the offset that marks an absent nonzero)
-    const bool paced = g_log2 >= 4 && !SDD && b_bytes >= kPacedBytes;
+    const bool full = g_log2 >= 5 && x.n_dense * (int64_t)sizeof(T) * 8 >= int64_t(16 * 7) << g_log2;
+    const bool paced = g_log2 >= 4 && !SDD && b_bytes >= (full ? kPacedWideBytes : kPacedBytes);
     if (g_log2 >= 2 && !paced && b_bytes <= (int64_t(1) << 32) - 1 - x.ldb * (int64_t)sizeof(T)) {
       if constexpr (SDD) {
         if (x.n_dense % VEC != 0) {

@@ -63,3 +63,22 @@ def test_ragged_width_keeps_infinities(device):
     used = torch.zeros(k, dtype=torch.bool, device=device)
     used[idx.long()] = True
     assert torch.all(torch.isposinf(dB[used][:, 3])) and torch.isfinite(dB[used][:, [0, 1, 2, 4]]).all()
+
+
+@pytest.mark.parametrize("n", [111, 112, 128])
+@pytest.mark.parametrize("rows", [49151, 49152, 56173])  # B of 24 MiB at 128 columns, at 112
+def test_spmm_where_wide_rows_change_kernels(device, rows, n):
+    """Dense operands on either side of 24 MiB whose rows fill their lane group or not."""
+    g = torch.Generator(device="cpu").manual_seed(rows + n)
+    lengths = torch.randint(0, 40, (700,), generator=g)
+    lengths[3] = 900  # segments
+    ptr = torch.zeros(701, dtype=torch.int32)
+    ptr[1:] = lengths.cumsum(0)
+    idx = torch.randint(0, rows, (int(ptr[-1]),), generator=g, dtype=torch.int32)
+    val = torch.randn(idx.numel(), generator=g)
+    B = torch.randn(rows, n, generator=g)
+    h = fs.CsrMatrix(idx.to(device), ptr.to(device), (700, rows)).handle
+    C = h.spmm(val.to(device), B.to(device)).cpu().double()
+    row = torch.repeat_interleave(torch.arange(700), lengths)
+    ref = torch.zeros(700, n, dtype=torch.float64).index_add_(0, row, val.double()[:, None] * B.double()[idx.long()])
+    assert (C - ref).abs().max() <= 1e-5 * ref.abs().max()
