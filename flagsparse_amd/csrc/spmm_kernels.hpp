@@ -338,13 +338,16 @@ constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : 8) : (SDD ? 4 : (ELEM == 2 ?
 // and value to the group.  A wave load costs the CU's address unit 18 clocks
 // whatever its lanes ask for (measured: all lanes, half masked off, half out
 // of range), so two of every three loads, and the offset arithmetic of every
-// lane, are what goes.  Nonzeros past a row's end have their B row outside the
-// buffer: it reads as zeros without memory traffic, so nothing is masked and
-// no load is repeated, and the batches of UNROLL rows that no lane needs are
-// skipped.  Vector instructions per launch fell from 45.2 to 24.1 million and
-// loads from 6.1 to 2.6 million (262144^2, N = 64).  100003 x 70001 f64,
-// N = 75: 290 -> 242 us; 1024-matrix batch, N = 32: 686 -> 664 us;
-// 200000-node graph, bf16 N = 128: 89 -> 86 us, its backward 144 -> 141 us.
+// lane, are what goes.  Nonzeros past a row's end read as value zero and have
+// their B row outside the buffer: it reads as zeros without memory traffic, so
+// nothing is masked and no load is repeated, and the batches of UNROLL rows
+// that no lane needs are skipped.  That takes both zeros: the next rows'
+// nonzeros are loaded in the wave's last trip and no sooner, or an infinite
+// value among them would meet the zeros of a row that has ended.  Vector
+// instructions per launch fell from 45.2 to 24.1 million and loads from 6.1 to
+// 2.6 million (262144^2, N = 64).  100003 x 70001 f64, N = 75: 290 -> 242 us;
+// 1024-matrix batch, N = 32: 686 -> 664 us; 200000-node graph, bf16 N = 128:
+// 89 -> 86 us, its backward 144 -> 141 us.
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool PERM,
           bool SDD, bool TAIL>
 __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cast<int>(sizeof(T))>)) void spmm_bins_kernel(
@@ -451,8 +454,9 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = A(0);
     P p = beg + slot;
-    bool prefetched = false;  // wave-uniform
-    while (__ballot(p < end) != 0) {  // wave-uniform: every lane takes part in the broadcasts
+    bool more = __ballot(p < end) != 0;  // wave-uniform: every lane takes part in the broadcasts
+    if (!more && has_next) trip(beg_n + slot, end_n, c, a, pq);
+    while (more) {
       O off[kRegs];
       A av[kRegs];
 #pragma unroll
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
         if constexpr (PERM) a[r] = data_b.load(ok ? static_cast<O>(pq[r]) : kAbsent);
       }
       const P pn = p + (static_cast<P>(kTrip) << s_log2);
-      const bool same = pn < end;
+      more = __ballot(pn < end) != 0;
       IT cn[kRegs];
       TV an[kRegs];
       QT pqn[kRegs];
@@ -477,11 +481,12 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
           b[u] = __builtin_bit_cast(
               V, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bcast<LANES, n % LANES>(off[n / LANES]) + col_off, 0, 0));
         });
-        // prefetch: the next trip of this item, else the first trip of the
-        // next.  Unconditional (with nothing next it touches no memory): under
-        // a branch the compiler could not count the loads in flight, and the
-        // last B row of the batch would wait for the prefetch too.
-        if constexpr (u0 == 0) trip(same ? pn : beg_n + slot, same ? end : end_n, cn, an, pqn);
+        // prefetch: the next trip of the wave's items, after the last one the
+        // first trip of the next items.  Unconditional (past an item's end, and
+        // with nothing next, it touches no memory): under a branch the compiler
+        // could not count the loads in flight, and the last B row of the batch
+        // would wait for the prefetch too.
+        if constexpr (u0 == 0) trip(more ? pn : beg_n + slot, more ? end : end_n, cn, an, pqn);
         if constexpr (u0 == 0) {
 #pragma unroll
           for (int r = 0; r < kRegs; ++r) av[r] = static_cast<A>(a[r]);
@@ -523,9 +528,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
         if constexpr (PERM || SDD) pq[r] = pqn[r];
       }
       p = pn;
-      prefetched = true;
     }
-    if (!prefetched && has_next) trip(beg_n + slot, end_n, c, a, pq);
     // Sum the S slots of a row: lanes that differ only in the slot bits.
     for (int j = 0; j < s_log2; ++j) {
 #pragma unroll
