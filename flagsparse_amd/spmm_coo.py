@@ -172,14 +172,11 @@ class _CanonicalCoo:
         """C = op(A) B in the requested layout (row-major kernel): B and C in
         the input dtype, products and sums in the values' compute dtype."""
         n_rows = self.shape[0]
-        B_row = B.contiguous().resolve_neg()
-        # the kernel writes a contiguous `out` itself unless it is B's own
-        # memory; an `out` in the autograd graph gets copy_'s checks
-        direct = (out if out is not None and out.is_contiguous() and not out.requires_grad
-                  and out.untyped_storage().data_ptr() != B_row.untyped_storage().data_ptr() else None)
-        C_row = self.handle.spmm(self.data, B_row, out=direct)
+        C_row = self.handle.spmm(self.data, B.contiguous().resolve_neg())
         if out is not None:
-            return out if direct is not None else out.copy_(C_row)
+            # copy_ and not the kernel writes `out`: it knows views that negate,
+            # tensors of other classes, tangents and the version that backward checks
+            return out.copy_(C_row)
         if dense_layout == "col":
             C = _empty_dense_layout((n_rows, int(B.shape[1])), B.dtype, C_row.device, "col")
             C.copy_(C_row)
