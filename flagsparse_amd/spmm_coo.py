@@ -68,6 +68,13 @@ def _materialize_dense_layout(tensor, layout):
     return out
 
 
+def _stride_in(tensor, dtype):
+    """Strides that the reference's meta reports: those of the operand in the
+    compute dtype, whose conversion drops the gaps of a padded one."""
+    t = torch.empty_strided(tensor.shape, tensor.stride(), dtype=tensor.dtype, device="meta").to(dtype)
+    return tuple(int(v) for v in t.stride())
+
+
 def _check_coo_ranges(row, col, n_rows, n_cols, nnz):
     """The nnz / index checks of spmm_coo.py:700-718 (same order and messages)."""
     if nnz > _INDEX_LIMIT_INT32:
@@ -453,7 +460,7 @@ def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, o
             "compute_ms": compute_ms,
             "op_total_ms": op_total_ms,
             "dense_layout": dense_layout,
-            "b_stride": tuple(int(v) for v in B.stride()),
+            "b_stride": _stride_in(B, compute_dtype),
             "c_stride": tuple(int(v) for v in C.stride()),
             "output_layout": _dense_layout_name(C),
         }
