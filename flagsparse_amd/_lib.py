@@ -217,10 +217,15 @@ def ptr(t):
 
 
 def stream_ptr(device=None):
-    """The current stream of `device` as an address.  The raw query: a
-    torch.cuda.Stream object per launch costs more than the launch's argument
-    conversion."""
-    index = None if device is None else device.index
+    """The current stream of `device` (None: the current device) as an address.
+    The raw query: a torch.cuda.Stream object per launch costs more than the
+    launch's argument conversion.  A device other than a GPU is refused: the
+    launch that asks would read its addresses on the GPU."""
+    if device is None:
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
+    index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
