@@ -6,11 +6,13 @@
 // one 1024-thread workgroup: at that size the work is a few microseconds and
 // every further launch costs as much as all of it (an unprepared SpMM call of
 // 4096 power-law rows, 65536 nonzeros, N = 32: 239 us with eight plan launches,
-// six copies and a second readback for the segments, 78 us now).  Larger ones take a counting pass over rows and columns (a
-// workgroup per 1024 rows, per-workgroup results instead of atomics, so
-// nothing has to be cleared first), one workgroup that reduces and scans the
-// counts, the stable scatter of the row ids and one workgroup that writes the
-// segments.
+// six copies and a second readback for the segments, 78 us now).  Larger ones
+// take a counting pass over rows and columns (a workgroup per 1024 rows,
+// per-workgroup results instead of atomics, so nothing has to be cleared
+// first), one workgroup that reduces and scans the counts, the stable scatter
+// of the row ids, one workgroup that scans the long rows' segment counts, and
+// a thread per segment (20000 rows and one of 16 M nonzeros: 96 us, 39 ms with
+// one thread per row).
 //
 // The structure is not trusted: lengths are taken as they come, and every
 // write is bounded by the sizes the caller passes.
@@ -109,12 +111,13 @@ __device__ __forceinline__ int64_t block_scan(int64_t v, int64_t* s_wave, int64_
   return before + v;
 }
 
-// Segments of the long rows rows[first, n_rows): row i of them is cut evenly
-// into ceil(len / seg_len) segments.  One workgroup.
-template <typename PT>
-__device__ __forceinline__ void write_segments(const PT* __restrict__ indptr, int64_t n_rows, int64_t first,
-                                               int64_t seg_len, const build_out& out, int64_t* s_wave,
-                                               int64_t* n_segments) {
+// Segment ranges of the long rows rows[first, n_rows): row i of them is cut
+// evenly into ceil(len / seg_len) segments.  One workgroup; put(at, n, row, b,
+// len) is called by all of its lanes together, n = 0 for lanes without a row.
+template <typename PT, typename F>
+__device__ __forceinline__ void scan_segments(const PT* __restrict__ indptr, int64_t n_rows, int64_t first,
+                                              int64_t seg_len, const build_out& out, int64_t* s_wave,
+                                              int64_t* n_segments, F&& put) {
   int64_t n_long = n_rows - first;
   if (n_long > out.max_long) n_long = out.max_long;
   int64_t carry = 0;
@@ -132,19 +135,41 @@ __device__ __forceinline__ void write_segments(const PT* __restrict__ indptr, in
     }
     int64_t total;
     const int64_t at = carry + block_scan(n, s_wave, total) - n;
-    if (live) {
-      out.long_seg_ptr[i] = at;
-      for (int64_t j = 0; j < n && at + j < out.max_segments; ++j) {
-        out.seg_row[at + j] = static_cast<int32_t>(row);
-        out.seg_begin[at + j] = b + len * j / n;
-        out.seg_end[at + j] = b + len * (j + 1) / n;
-      }
-    }
+    if (live) out.long_seg_ptr[i] = at;
+    put(at, n, row, b, len);
     carry += total;
   }
   if (threadIdx.x == 0) {
     if (n_long > 0) out.long_seg_ptr[n_long] = carry;
     *n_segments = carry;
+  }
+}
+
+// Segment j of the n that a row's [b, b + len) is cut into; `at` is below max_segments.
+__device__ __forceinline__ void write_segment(const build_out& out, int64_t at, int64_t j, int64_t n, int64_t row,
+                                              int64_t b, int64_t len) {
+  out.seg_row[at] = static_cast<int32_t>(row);
+  out.seg_begin[at] = b + len * j / n;
+  out.seg_end[at] = b + len * (j + 1) / n;
+}
+
+// One wave writes the segments of its lanes' rows: a lane by itself for a row
+// of few, all lanes together for a row of many (one lane took 0.6 us a segment,
+// two divisions and three stores after one another).
+constexpr int kLaneSegments = 4;
+__device__ __forceinline__ void write_segments(const build_out& out, int64_t at, int64_t n, int64_t row, int64_t b,
+                                               int64_t len) {
+  const bool few = n <= kLaneSegments;
+  if (few) {
+    for (int64_t j = 0; j < n && at + j < out.max_segments; ++j) write_segment(out, at + j, j, n, row, b, len);
+  }
+  for (uint64_t left = __ballot(!few); left != 0; left &= left - 1) {  // wave-uniform
+    const int from = __ffsll(static_cast<unsigned long long>(left)) - 1;
+    const int64_t at_w = __shfl(at, from), n_w = __shfl(n, from), row_w = __shfl(row, from), b_w = __shfl(b, from),
+                  len_w = __shfl(len, from);
+    for (int64_t j = threadIdx.x & 63; j < n_w && at_w + j < out.max_segments; j += 64) {
+      write_segment(out, at_w + j, j, n_w, row_w, b_w, len_w);
+    }
   }
 }
 
@@ -209,7 +234,10 @@ __global__ __launch_bounds__(kBuildThreads) void plan_small_kernel(const PT* __r
     }
     __syncthreads();  // the last one also orders the row ids before their reads below
   }
-  write_segments(indptr, n_rows, s_off[n_bins - 1], seg_len, out, s_wave, &out.meta[kMetaStats + n_bins + 1]);
+  scan_segments(indptr, n_rows, s_off[n_bins - 1], seg_len, out, s_wave, &out.meta[kMetaStats + n_bins + 1],
+                [&](int64_t at, int64_t n, int64_t row, int64_t b, int64_t len) {
+                  write_segments(out, at, n, row, b, len);
+                });
 }
 
 // Workgroup b counts the bins of rows [1024 b, 1024 (b + 1)) into
@@ -288,11 +316,39 @@ __global__ __launch_bounds__(kBuildThreads) void plan_reduce_kernel(const PT* __
 }
 
 template <typename PT>
-__global__ __launch_bounds__(kBuildThreads) void plan_segments_kernel(const PT* __restrict__ indptr, int64_t n_rows,
-                                                                      int n_bins, int64_t seg_len, build_out out) {
+__global__ __launch_bounds__(kBuildThreads) void plan_ranges_kernel(const PT* __restrict__ indptr, int64_t n_rows,
+                                                                    int n_bins, int64_t seg_len, build_out out) {
   __shared__ int64_t s_wave[kBuildWaves];
-  write_segments(indptr, n_rows, out.meta[kMetaStats + n_bins - 1], seg_len, out, s_wave,
-                 &out.meta[kMetaStats + n_bins + 1]);
+  scan_segments(indptr, n_rows, out.meta[kMetaStats + n_bins - 1], seg_len, out, s_wave,
+                &out.meta[kMetaStats + n_bins + 1], [](int64_t, int64_t, int64_t, int64_t, int64_t) {});
+}
+
+// The segments themselves, a thread each: thread s finds its row in the ranges.
+template <typename PT>
+__global__ __launch_bounds__(FSP_WG_THREADS) void plan_segments_kernel(const PT* __restrict__ indptr, int64_t n_rows,
+                                                                       int n_bins, build_out out) {
+  const int64_t first = out.meta[kMetaStats + n_bins - 1];
+  int64_t n_long = n_rows - first;
+  if (n_long > out.max_long) n_long = out.max_long;
+  int64_t n_seg = out.meta[kMetaStats + n_bins + 1];
+  if (n_seg > out.max_segments) n_seg = out.max_segments;
+  if (n_long <= 0) return;
+  for (int64_t s = static_cast<int64_t>(blockIdx.x) * FSP_WG_THREADS + threadIdx.x; s < n_seg;
+       s += static_cast<int64_t>(gridDim.x) * FSP_WG_THREADS) {
+    int64_t lo = 0, hi = n_long;  // long_seg_ptr[lo] <= s < long_seg_ptr[hi]
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (out.long_seg_ptr[mid] <= s) {
+        lo = mid;
+      } else {
+        hi = mid;
+      }
+    }
+    const int64_t at = out.long_seg_ptr[lo], n = out.long_seg_ptr[lo + 1] - at;
+    const int64_t row = out.rows[first + lo];
+    const int64_t b = static_cast<int64_t>(indptr[row]);
+    write_segment(out, s, s - at, n, row, b, static_cast<int64_t>(indptr[row + 1]) - b);
+  }
 }
 
 static inline int64_t build_row_blocks(int64_t n_rows) {
@@ -306,6 +362,10 @@ static inline int64_t build_blocks(int64_t n_rows, int64_t nnz) {
   if (c > 1024) c = 1024;
   const int64_t r = build_row_blocks(n_rows);
   return c > r ? c : r;
+}
+static inline int64_t segment_blocks(int64_t max_segments) {
+  const int64_t b = ceil_div(max_segments, int64_t(FSP_WG_THREADS));
+  return b < 2048 ? b : 2048;
 }
 
 }  // namespace fsp
@@ -338,6 +398,9 @@ int fsp_csr_build_plan(int32_t indptr_type, const void* indptr_dev, int32_t inde
   if (n_bins > 0 && n_rows > (int64_t)INT32_MAX) {
     return fail(FSP_ERR_ARG, "fsp_csr_build_plan: n_rows exceeds int32 row ids");
   }
+  // without columns to look at, the nonzeros only count as segments: 4096 of
+  // 256 for one wave at most
+  const bool small = n_rows <= kSmallRows && nnz <= (indices_dev == nullptr ? 8 * kSmallNnz : kSmallNnz);
   if (indices_dev == nullptr) nnz = 0;  // no columns to look at
   bin_bounds bb;
   for (int b = 0; b < FSP_MAX_BINS; ++b) bb.upper[b] = INT64_MAX;
@@ -345,7 +408,6 @@ int fsp_csr_build_plan(int32_t indptr_type, const void* indptr_dev, int32_t inde
   const build_out out{meta_dev, rows_dev, max_segments, seg_row_dev, seg_begin_dev, seg_end_dev, max_long,
                       long_seg_ptr_dev};
   const hipStream_t s = as_stream(stream);
-  const bool small = n_rows <= kSmallRows && nnz <= kSmallNnz;
   const int64_t row_blocks = build_row_blocks(n_rows);
   const int64_t blocks = build_blocks(n_rows, nnz);
   if (!small) {
@@ -378,8 +440,11 @@ int fsp_csr_build_plan(int32_t indptr_type, const void* indptr_dev, int32_t inde
                          ip, n_rows, n_bins, bb, counts, row_blocks, rows_dev);
       st = check_launch("bins_scatter");
       if (st) return st;
-      hipLaunchKernelGGL(plan_segments_kernel<PT>, dim3(1), dim3(kBuildThreads), 0, s, ip, n_rows, n_bins, seg_len,
-                         out);
+      hipLaunchKernelGGL(plan_ranges_kernel<PT>, dim3(1), dim3(kBuildThreads), 0, s, ip, n_rows, n_bins, seg_len, out);
+      st = check_launch("plan_ranges");
+      if (st || max_segments == 0) return st;
+      hipLaunchKernelGGL(plan_segments_kernel<PT>, dim3(static_cast<unsigned>(segment_blocks(max_segments))),
+                         dim3(FSP_WG_THREADS), 0, s, ip, n_rows, n_bins, out);
       return check_launch("plan_segments");
     });
   });
