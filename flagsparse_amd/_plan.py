@@ -25,7 +25,7 @@ The reference rebuilds its buckets with ``torch.nonzero`` on every call
 """
 
 import ctypes
-from dataclasses import dataclass, field
+from dataclasses import dataclass
 from functools import lru_cache
 
 import torch
@@ -187,10 +187,14 @@ class CsrPlan:
     n_long_rows: int
     row_len: int = 0  # > 0: every row has exactly this many nonzeros
     indptr_base: int = 0  # indptr[0] when row_len > 0
-    _structs: dict = field(default_factory=dict, init=False, repr=False, compare=False)
 
-    # The structs hold the addresses of this plan's own tensors: a copy, a pickle
+    # _structs: the C plans made so far.  They hold the addresses of this plan's
+    # own tensors, so a field that is assigned drops them, and a copy, a pickle
     # or a plan that was saved before there were any starts without them.
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        self.__dict__["_structs"] = {}
+
     def __getstate__(self):
         state = dict(self.__dict__)
         state.pop("_structs", None)
@@ -198,7 +202,7 @@ class CsrPlan:
 
     def __setstate__(self, state):
         self.__dict__.update(state)
-        self._structs = {}
+        self.__dict__["_structs"] = {}
 
     @property
     def bin_sizes(self):
@@ -223,7 +227,7 @@ class CsrPlan:
         region per XCD).  variant selects the SpMV loop (0 pipelined, 1 plain,
         2 plain and 3 pipelined with x staged in LDS, 4 vector chunks with x
         in LDS)."""
-        key = (max_blocks, xcd_groups, variant, self.row_len, self.indptr_base)
+        key = (max_blocks, xcd_groups, variant)
         base = self._structs.get(key)
         if base is None:
             base = self._structs[key] = self._struct(max_blocks, xcd_groups, variant)
