@@ -48,14 +48,17 @@ def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes):
 
 
 class CsrHandle:
-    __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "_plans", "_csc", "_csc_plans")
+    __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "row_nnz", "_plans", "_csc", "_csc_plans")
 
-    def __init__(self, indices, indptr, shape):
+    def __init__(self, indices, indptr, shape, row_nnz=None):
+        """row_nnz: nonzeros of the rows, where `indptr` is a range of the row
+        pointer that `indices` belongs to (it sizes the plan's buffers)."""
         self.indices = indices
         self.indptr = indptr
         self.shape = (int(shape[0]), int(shape[1]))
         self.n_rows, self.n_cols = self.shape
         self.nnz = int(indices.numel())
+        self.row_nnz = self.nnz if row_nnz is None else int(row_nnz)
         self._plans = {}
         self._csc = None
         self._csc_plans = {}
@@ -64,7 +67,7 @@ class CsrHandle:
     def plan(self, config):
         p = self._plans.get(config)
         if p is None:
-            p = _plan.build_plan(self.indptr, self.n_rows, config, self.nnz)
+            p = _plan.build_plan(self.indptr, self.n_rows, config, self.row_nnz)
             self._plans[config] = p
         return p
 

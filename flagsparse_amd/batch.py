@@ -350,7 +350,7 @@ class CsrBatch:
                 # the matrix's rows of the packed block-diagonal CSR: a row
                 # range of the packed row pointer over the packed column ids
                 # (global columns, the packed arrays' own alignment)
-                hg = CsrHandle(self.indices, self.indptr[r0: r1 + 1], (r1 - r0, self.total_cols))
+                hg = CsrHandle(self.indices, self.indptr[r0: r1 + 1], (r1 - r0, self.total_cols), n1 - n0)
                 mats.append((h, hg, r0, r1, n0, n1, c0, c1))
             self._per_matrix = mats
         return self._per_matrix
