@@ -169,7 +169,7 @@ def _index_code(t):
     return _lib.index_code(t.dtype)
 
 
-@dataclass
+@dataclass(init=False)
 class CsrPlan:
     """Device work plan of one index structure (see module docstring)."""
 
@@ -188,12 +188,20 @@ class CsrPlan:
     row_len: int = 0  # > 0: every row has exactly this many nonzeros
     indptr_base: int = 0  # indptr[0] when row_len > 0
 
+    def __init__(self, config, n_rows, rows, bin_counts, identity, seg_row, seg_begin, seg_end, long_rows, long_seg_ptr,
+                 n_segments, n_long_rows, row_len=0, indptr_base=0):
+        # (an assignment each would cost an unprepared call 3 us)
+        self.__dict__.update(
+            config=config, n_rows=n_rows, rows=rows, bin_counts=bin_counts, identity=identity, seg_row=seg_row,
+            seg_begin=seg_begin, seg_end=seg_end, long_rows=long_rows, long_seg_ptr=long_seg_ptr,
+            n_segments=n_segments, n_long_rows=n_long_rows, row_len=row_len, indptr_base=indptr_base, _structs={})
+
     # _structs: the C plans made so far.  They hold the addresses of this plan's
     # own tensors, so a field that is assigned drops them, and a copy, a pickle
     # or a plan that was saved before there were any starts without them.
     def __setattr__(self, name, value):
         object.__setattr__(self, name, value)
-        self.__dict__["_structs"] = {}
+        object.__setattr__(self, "_structs", {})
 
     def __getstate__(self):
         state = dict(self.__dict__)
@@ -201,8 +209,7 @@ class CsrPlan:
         return state
 
     def __setstate__(self, state):
-        self.__dict__.update(state)
-        self.__dict__["_structs"] = {}
+        self.__dict__.update(state, _structs={})
 
     @property
     def bin_sizes(self):
