@@ -30,21 +30,20 @@ def _acc_dtype(dtype):
 _PERMUTED_BYTES = 2 << 20
 
 
-def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes):
+def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes, backward=False):
     """True where the transposed kernels read data[perm[q]] beside their
     gathers of the dense rows (ld x rows) instead of after a pass that gathers
-    the values: where the kernel's lanes share their nonzeros (the conditions
-    of csrc/spmm_kernels.hpp; elsewhere every lane would read it for itself)
-    and the values stay in the L2s.  Graphs of mean degree 14, N = 64, f32:
-    16000 nodes (0.9 MB of values) 15.1 against 20.9 us, 32000 nodes 19.6
-    against 22.1, 64000 nodes (3.6 MB) 37.0 against 35.3, 128000 nodes 78 against
-    68, where each of those reads is another 128 bytes across the fabric."""
+    the values: where the kernel's lanes share their nonzeros (elsewhere every
+    lane would read it for itself) and the values stay in the L2s.  Graphs of
+    mean degree 14, N = 64, f32: 16000 nodes (0.9 MB of values) 15.1 against
+    20.9 us, 32000 nodes 19.6 against 22.1, 64000 nodes (3.6 MB) 37.0 against
+    35.3, 128000 nodes 78 against 68, where each of those reads is another 128
+    bytes across the fabric."""
     elem = data.element_size()
-    dense = rows * ld * elem
-    paced = (24 if lanes >= 32 and n_dense * elem * 8 >= 16 * 7 * lanes else 64) << 20
-    return (perm.numel() * elem <= _PERMUTED_BYTES and lanes >= 4 and n_dense >= 16 // elem
-            and perm.dtype == torch.int32 and dense + ld * elem < 1 << 32 and n_out * n_dense * elem < 1 << 32
-            and (lanes < 16 or dense < paced))
+    return (perm.numel() * elem <= _PERMUTED_BYTES and perm.dtype == torch.int32
+            and rows * ld * elem < 1 << 32 and n_out * n_dense * elem < 1 << 32
+            and _lib.load().fsp_spmm_shares_nonzeros(_lib.value_code(data.dtype), lanes, n_dense, ld, rows,
+                                                     backward) == 1)
 
 
 class CsrHandle:
@@ -181,9 +180,8 @@ class CsrHandle:
         colptr, rowind, perm = self.csc()
         plan = self.csc_plan(cfg)
         name = "fsp_spmm_csr_trans_sddmm"
-        # (this kernel is not paced at the wide groups' lower size)
-        if self.nnz and not _permuted_in_kernel(data, perm, int(dC.stride(0)), self.n_rows, self.n_cols, n_dense,
-                                                min(G, 16)):
+        if self.nnz and not _permuted_in_kernel(data, perm, int(dC.stride(0)), self.n_rows, self.n_cols, n_dense, G,
+                                                True):
             data = gather_values(data, perm)
         elif self.nnz:
             name = "fsp_spmm_csr_trans_sddmm_perm"

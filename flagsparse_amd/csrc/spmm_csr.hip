@@ -109,6 +109,13 @@ extern "C" int fsp_spmm_csr(int32_t value_type, int32_t index_type, int32_t indp
                     B_dev, ldb, C_dev, ldc, n_rows, n_dense, nnz, b_rows, lanes_n, plan, stream);
 }
 
+extern "C" int fsp_spmm_shares_nonzeros(int32_t value_type, int32_t lanes_n, int64_t n_dense, int64_t ldb,
+                                        int64_t b_rows, int32_t backward) {
+  const int64_t elem = value_type == FSP_F64 ? 8 : (value_type == FSP_F32 ? 4 : 2);
+  if (lanes_n < 1 || lanes_n > 64 || !is_pow2(lanes_n) || n_dense < 16 / elem || ldb < n_dense || b_rows < 0) return 0;
+  return spmm_shares_nonzeros(elem, ilog2(lanes_n), n_dense, ldb, b_rows, backward != 0) ? 1 : 0;
+}
+
 extern "C" int fsp_spmm_csr_wide(int32_t dense_type, int32_t index_type, int32_t indptr_type, const void* indptr_dev,
                                  const void* indices_dev, const void* data_dev, const void* B_dev, int64_t ldb,
                                  void* C_dev, int64_t ldc, int64_t n_rows, int64_t n_dense, int64_t nnz,

@@ -294,20 +294,44 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
 // touches no memory.
 constexpr uint32_t kAbsent = ~0u;
 
-// B of at least twice the eight 4 MiB L2s, read in rows of 256 bytes or more:
-// nearly every gather crosses the fabric, and more of them in flight lowers its
-// throughput (262144^2, f32: N = 64 233 us with spmm_bins_kernel, 227 us with
-// five workgroups per CU, 228 us with spmm_slots_kernel; N = 160 558 against
-// 543 us).  Below that size the faster issue wins (200000-node graph, bf16
-// N = 128: 86 against 89 us; 50000 nodes, f32 N = 64: 24 against 26 us).
-// Rows of 512 bytes or more that use nearly every lane of their group are paced
-// from 24 MiB on: a wave load brings 1 KiB there and issuing is no bound (slots
-// against bins: 100000^2, f64 N = 64 166 / 173 us, f32 N = 128 171 / 174.5; 50000^2,
-// 25 MB of B, f32 N = 128 80.8 / 83.8, bf16 N = 256 84.8 / 87.5; 10 MB, f64 N = 64
-// 37.8 / 32.8).  With fewer lanes in use the faster issue wins (f64 N = 75, 42 MB
-// of B, 38 of 64 lanes: 290 / 242).
-constexpr int64_t kPacedBytes = int64_t(64) << 20;
-constexpr int64_t kPacedWideBytes = int64_t(24) << 20;
+// Where B's rows come across the fabric, more gathers in flight lower its
+// throughput, and the loop whose lanes load their nonzeros each for themselves
+// (spmm_slots_kernel) paces them; below that the faster issue of
+// spmm_bins_kernel wins.  Time of the former over the latter, int32 indices,
+// rows of power-law length (mean 24) with uniform columns / graphs with hub
+// columns (mean 14), which the caches keep:
+//                                   24 MiB       40           48           56           64           96
+//   16 lanes  f32  N =  64      0.995/1.064  0.986/1.030  0.987/1.011  0.979/1.016  0.989/1.007  0.989/1.003
+//             bf16 N = 128      1.012/1.096  1.009/1.040  0.992/1.035  0.986/1.040  1.004/1.027  0.991/1.021
+//   32 lanes  f32  N = 128      0.995/1.057  0.990/1.027  0.963/1.007  0.975/1.015  0.983/0.992  0.978/0.984
+//             f64  N =  64      1.014/1.106  0.975/1.050  0.953/1.038  0.960/1.034  0.972/1.020  0.967/1.003
+//   64 lanes  f64  N = 128      1.085/1.249  1.007/1.121  0.994/1.072  0.994/1.044  0.981/1.086  0.976/1.014
+//   38 of 64  f64  N =  75      1.072/1.324  1.058/1.201  1.066/1.160  1.033/1.128  1.047/1.135  1.017/1.099
+// The limits lie where what one pattern gains is what the other loses: 48 MiB
+// for rows that fill a group of 32 lanes or more (seven lanes in eight), 56 MiB
+// for other groups of 16 or 32.  A 64-lane group with idle lanes is not paced
+// (38 of 64 up to 400 MiB: 1.01-1.14), nor are groups of 8 lanes (f32 N = 32, 32
+// to 128 MiB: 1.00-1.02, f64 N = 16 0.99-1.08) and the backward (32 to 256 MiB:
+// f32 N = 64 1.01-1.12, bf16 N = 128 1.01-1.08, f64 N = 64 1.09-1.27).
+constexpr int64_t kPacedBytes = int64_t(56) << 20;
+constexpr int64_t kPacedFullBytes = int64_t(48) << 20;
+static inline bool spmm_paced(int64_t elem_bytes, int g_log2, int64_t n_dense, int64_t b_bytes, bool backward) {
+  const bool full = n_dense * elem_bytes * 8 >= int64_t(16 * 7) << g_log2;
+  if (backward || g_log2 < 4 || (g_log2 == 6 && !full)) return false;
+  return b_bytes >= (g_log2 >= 5 && full ? kPacedFullBytes : kPacedBytes);
+}
+
+// Whether a launch of whole vectors with 32-bit offsets shares its nonzeros
+// between lanes (spmm_bins_kernel): groups of four lanes or more whose gathers
+// are not paced.  (B's bytes and a row stay below the offset that marks an
+// absent nonzero.)
+static inline bool spmm_shares_nonzeros(int64_t elem_bytes, int g_log2, int64_t n_dense, int64_t ldb, int64_t b_rows,
+                                        bool backward) {
+  const int64_t b_bytes = b_rows * ldb * elem_bytes;
+  return g_log2 >= 2 && b_bytes <= (int64_t(1) << 32) - 1 - ldb * elem_bytes &&
+         !spmm_paced(elem_bytes, g_log2, n_dense, b_bytes, backward);
+}
+
 template <typename E>
 struct buffer {
   __amdgpu_buffer_rsrc_t rsrc;
@@ -636,10 +660,7 @@ static void launch_bins(const spmm_args& x, dim3 grid, int g_log2, typename acc_
         bins(spmm_bins_kernel<T, TV, IT, PT, QT, VEC, UNROLL, 4, PERM, SDD, TAIL>);
       }
     };
-    // (b_bytes + a row stays below the offset that marks an absent nonzero)
-    const bool full = g_log2 >= 5 && x.n_dense * (int64_t)sizeof(T) * 8 >= int64_t(16 * 7) << g_log2;
-    const bool paced = g_log2 >= 4 && !SDD && b_bytes >= (full ? kPacedWideBytes : kPacedBytes);
-    if (g_log2 >= 2 && !paced && b_bytes <= (int64_t(1) << 32) - 1 - x.ldb * (int64_t)sizeof(T)) {
+    if (spmm_shares_nonzeros(sizeof(T), g_log2, x.n_dense, x.ldb, x.b_rows, SDD)) {
       if constexpr (SDD) {
         if (x.n_dense % VEC != 0) {
           width(std::true_type{});

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FSP_ABI_VERSION 18
+#define FSP_ABI_VERSION 19
 #define FSP_MAX_BINS 8
 
 typedef enum fsp_value_type {
@@ -229,6 +229,15 @@ int fsp_spmm_csr(int32_t value_type, int32_t index_type, int32_t indptr_type,
                  const void* B_dev, int64_t ldb, void* C_dev, int64_t ldc,
                  int64_t n_rows, int64_t n_dense, int64_t nnz, int64_t b_rows,
                  int32_t lanes_n, const fsp_csr_plan* plan, void* stream);
+
+/* 1 if a product over `b_rows` dense rows of `n_dense` value_type elements
+ * (leading dimension ldb), `lanes_n` lanes along them, loads each nonzero in
+ * one lane that shares it with its group, 0 if every lane loads it (or the
+ * arguments are no product).  The rule of fsp_spmm_csr and, with `backward`, of
+ * fsp_spmm_csr_trans_sddmm where every array is below 4 GiB: a value read through
+ * a permutation then costs one read per nonzero, else one per lane. */
+int fsp_spmm_shares_nonzeros(int32_t value_type, int32_t lanes_n, int64_t n_dense, int64_t ldb, int64_t b_rows,
+                             int32_t backward);
 
 /* fsp_spmm_csr without a permutation whose values are wider than the dense
  * operands: `dense_type` FSP_F32 takes f64 values and sums in f64, FSP_BF16 /
