@@ -11,6 +11,8 @@ _permuted_in_kernel).  The transposed SpMV always reads through ``perm``.  All l
 libflagsparse_hip.so.
 """
 
+from functools import lru_cache
+
 import torch
 
 from . import _lib, _plan
@@ -42,8 +44,12 @@ def _permuted_in_kernel(data, perm, ld, rows, n_out, n_dense, lanes, backward=Fa
     elem = data.element_size()
     return (perm.numel() * elem <= _PERMUTED_BYTES and perm.dtype == torch.int32
             and rows * ld * elem < 1 << 32 and n_out * n_dense * elem < 1 << 32
-            and _lib.load().fsp_spmm_shares_nonzeros(_lib.value_code(data.dtype), lanes, n_dense, ld, rows,
-                                                     backward) == 1)
+            and _shares_nonzeros(_lib.value_code(data.dtype), lanes, n_dense, ld, rows, backward))
+
+
+@lru_cache(maxsize=256)
+def _shares_nonzeros(value_code, lanes, n_dense, ld, rows, backward):
+    return _lib.load().fsp_spmm_shares_nonzeros(value_code, lanes, n_dense, ld, rows, backward) == 1
 
 
 class CsrHandle:
