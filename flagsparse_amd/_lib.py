@@ -217,17 +217,29 @@ def ptr(t):
     return t.data_ptr() if t.numel() > 0 else None
 
 
-def stream_ptr(device=None):
-    """The current stream of `device` (None: the current device) as an address.
-    The raw query: a torch.cuda.Stream object per launch costs more than the
-    launch's argument conversion.  A device other than a GPU is refused: the
-    launch that asks would read its addresses on the GPU."""
+_gpu_index = {}  # torch.device with an index -> that index, GPUs only
+
+
+def _index_of(device):
+    """The index of a GPU; another device is refused, since the launch that
+    asks would read its addresses on the GPU."""
     if device is None:
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        return torch.cuda.current_device()
     if device.type != "cuda":
         raise ValueError(f"Expected a cuda device, but got: {device}")
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if device.index is None:
+        return torch.cuda.current_device()
+    _gpu_index[device] = device.index
+    return device.index
+
+
+def stream_ptr(device=None):
+    """The current stream of `device` (None: the current device) as an address.
+    The raw query, and the device's type looked at once: a torch.cuda.Stream
+    object per launch costs more than the launch's argument conversion, and the
+    type's name 0.2 us."""
+    index = _gpu_index.get(device)
+    return torch._C._cuda_getCurrentRawStream(_index_of(device) if index is None else index)
 
 
 def device_arch():

@@ -33,3 +33,13 @@ def test_host_tensors(monkeypatch, call):
     h = CsrHandle(torch.tensor([0, 1, 2], dtype=torch.int32), torch.tensor([0, 1, 3], dtype=torch.int32), (2, 3))
     with pytest.raises(ValueError, match="cuda device"):
         call(h, torch.ones(3), torch.arange(3, dtype=torch.int32))
+
+
+def test_index_of_a_device(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 5)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index, raising=False)
+    for _ in range(2):
+        assert _lib.stream_ptr(torch.device("cuda:3")) == 103 and _lib.stream_ptr(torch.device("cuda:0")) == 100
+        assert _lib.stream_ptr(torch.device("cuda")) == _lib.stream_ptr() == 105
+        with pytest.raises(ValueError, match="cuda device"):
+            _lib.stream_ptr(torch.device("cpu:0"))
