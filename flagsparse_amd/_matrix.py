@@ -7,8 +7,8 @@ the index structure is cached, so a handle stays valid while the values change
 (training): a transposed SpMM reads a small value array through ``perm``
 (data[perm[q]]) inside its kernel and gathers a larger one into CSC order on
 every call (``fsp_gather`` into a buffer of the caching allocator, see
-_permuted_in_kernel).  The transposed SpMV always reads through ``perm``.  All launches go through the C ABI of
-libflagsparse_hip.so.
+_permuted_in_kernel).  The transposed SpMV always reads through ``perm``.  All
+launches go through the C ABI of libflagsparse_hip.so.
 """
 
 from functools import lru_cache

@@ -97,7 +97,8 @@ def spmv_wide_config():
     workgroup each.  f32, 100000 rows of 10 on average: power-law up to 4096 /
     with 20 rows of 9000, microseconds: one wave a row 15.6 / 20.4; a workgroup
     above 256: 11.2, above 512: 10.7 / 12.6, above 1024: 10.5 / 12.6, above 2048:
-    11.1."""
+    11.1.  The tuner's candidates have no such bin, so a tuned plan keeps one
+    wave a row."""
     base = spmv_config(long_threshold=SPMV_WIDE_ROW)
     return PlanConfig(base.lanes + (SPMV_WIDE_LANES,), base.uppers + (SPMV_LONG_THRESHOLD,), SPMV_SEG_LEN, SPMV_UNROLL)
 

@@ -486,9 +486,8 @@ __global__ __launch_bounds__(64 * WPG) void bsr_spmm_kernel(
 // block columns together and a wave that is ahead misses L2 while the others
 // hit what it brought in, so few waves with wide rows stay in step: 65536^2,
 // 40 blocks per row, N = 128, bf16 takes 56 us here (ROWS 2, TILES 8: 2048
-// waves) against 67 us with bsr_spmm_kernel's 16384 waves; four waves per block
-// row and 2 to 4 pairs in flight fetch 4.8 instead of 2.8 million lines of 128
-// bytes across the fabric and take 83-90 us.  fp8 48 -> 39 us; 20000^2, 20
+// waves; 2.7 million lines miss L2) against 67 us with bsr_spmm_kernel's 16384
+// waves; four waves per block row and 2 to 4 pairs in flight took 83-90 us.  fp8 48 -> 39 us; 20000^2, 20
 // blocks, N = 256: 25 -> 21 us; 65536^2, 20 blocks, N = 48: 37 -> 19 us.
 template <int KIND, typename BP, int TILES, int ROWS>
 __global__ __launch_bounds__(64) void bsr_spmm_sweep_kernel(

@@ -367,11 +367,12 @@ constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : 8) : (SDD ? 4 : (ELEM == 2 ?
 // nothing is masked and no load is repeated, and the batches of UNROLL rows
 // that no lane needs are skipped.  That takes both zeros: the next rows'
 // nonzeros are loaded in the wave's last trip and no sooner, or an infinite
-// value among them would meet the zeros of a row that has ended.  Vector
-// instructions per launch fell from 45.2 to 24.1 million and loads from 6.1 to
-// 2.6 million (262144^2, N = 64).  100003 x 70001 f64, N = 75: 290 -> 242 us;
-// 1024-matrix batch, N = 32: 686 -> 664 us; 200000-node graph, bf16 N = 128:
-// 89 -> 86 us, its backward 144 -> 141 us.
+// value among them would meet the zeros of a row that has ended.  Against
+// spmm_slots_kernel, vector instructions per launch fall from 44.6 to 23.7
+// million and loads from 6.0 to 2.6 million (262144 x 229376, f32 N = 64, either
+// side of the limit above).  100003 x 70001 f64, N = 75: 290 -> 240 us;
+// 1024-matrix batch, N = 32: 687 -> 665 us; 200000-node graph, bf16 N = 128, by
+// kernel: 84.6 -> 80.7 us, its backward 130.5 -> 127.1 us.
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool PERM,
           bool SDD, bool TAIL>
 __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cast<int>(sizeof(T))>)) void spmm_bins_kernel(

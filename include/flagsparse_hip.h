@@ -61,7 +61,8 @@ typedef struct fsp_bin {
 
 /* Work plan of one CSR (or CSC) matrix: rows binned by length, plus the
  * nnz-balanced split of rows longer than the last bin into segments.  All
- * arrays are device memory owned by the caller (built by fsp_csr_build_plan). */
+ * arrays are device memory owned by the caller (built by fsp_csr_build_plan, or
+ * with bins from fsp_csr_row_bins). */
 typedef struct fsp_csr_plan {
   int32_t n_bins;
   int32_t unroll;                 /* nonzeros per lane per loop trip (1..8) */
