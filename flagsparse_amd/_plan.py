@@ -377,6 +377,15 @@ def inspect_csr(indptr, indices, n_rows, nnz, config=None, meanwhile=None):
     return stats, plan
 
 
+def _copies(*tensors):
+    """Copies that are written when this returns, as everything else of a plan
+    is: the next launch may be on another stream."""
+    out = [t.clone() for t in tensors]
+    if out[0].is_cuda:
+        torch.cuda.current_stream(out[0].device).synchronize()
+    return out
+
+
 def _finish_plan(indptr, n_rows, config, arrays, row_len=0, indptr_base=0):
     """The plan from the arrays of _build for a valid CSR.
     row_len > 0 (every row that long, indptr[i] = indptr_base + i * row_len)
@@ -397,15 +406,15 @@ def _finish_plan(indptr, n_rows, config, arrays, row_len=0, indptr_base=0):
         long_rows = rows[off[nb - 1]: off[nb]]
         held = seg_begin.untyped_storage().nbytes()
         if held > _KEEP_BYTES and held > 8 * 8 * n_seg:  # few segments of what was provided for
-            rows, seg_row, long_rows = rows.clone(), seg_row.clone(), long_rows.clone()
-            seg_begin, seg_end, long_seg_ptr = seg_begin.clone(), seg_end.clone(), long_seg_ptr.clone()
+            rows, seg_row, long_rows, seg_begin, seg_end, long_seg_ptr = _copies(
+                rows, seg_row, long_rows, seg_begin, seg_end, long_seg_ptr)
     else:
         if n_long:
             raise RuntimeError("the row pointer holds more nonzeros than the plan was built for")
         seg_row = long_rows = torch.empty(0, dtype=torch.int32, device=device)
         seg_begin = seg_end = long_seg_ptr = torch.empty(0, dtype=torch.int64, device=device)
         if rows.untyped_storage().nbytes() > 4 * n_rows + _KEEP_BYTES:
-            rows = rows.clone()
+            rows, = _copies(rows)
     return CsrPlan(
         config=config,
         n_rows=n_rows,
