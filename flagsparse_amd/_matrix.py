@@ -72,7 +72,8 @@ class CsrHandle:
     def plan(self, config):
         p = self._plans.get(config)
         if p is None:
-            p = _plan.build_plan(self.indptr, self.n_rows, config, self.row_nnz)
+            nnz = getattr(self, "row_nnz", self.nnz)  # absent in a handle saved without it
+            p = _plan.build_plan(self.indptr, self.n_rows, config, nnz)
             self._plans[config] = p
         return p
 
