@@ -10,9 +10,14 @@
 // take a counting pass over rows and columns (a workgroup per 1024 rows,
 // per-workgroup results instead of atomics, so nothing has to be cleared
 // first), one workgroup that reduces and scans the counts, the stable scatter
-// of the row ids, one workgroup that scans the long rows' segment counts, and
-// a thread per segment (20000 rows and one of 16 M nonzeros: 96 us, 39 ms with
-// one thread per row).
+// of the row ids, and the workgroups that write the segments (20000 rows and
+// one of 16 M nonzeros: 77 us in all, 39 ms with a thread per row; 50000 rows of
+// 5000: 0.65 ms and 1.8).
+//
+// A launch more before the readback costs more than its run: with the ranges
+// and the segments in kernels of their own the host's wait outgrew the time that
+// it polls, and the first product on a new matrix of 9904 rows took 163 us
+// instead of 140.
 //
 // The structure is not trusted: lengths are taken as they come, and every
 // write is bounded by the sizes the caller passes.
@@ -111,13 +116,26 @@ __device__ __forceinline__ int64_t block_scan(int64_t v, int64_t* s_wave, int64_
   return before + v;
 }
 
-// Segment ranges of the long rows rows[first, n_rows): row i of them is cut
-// evenly into ceil(len / seg_len) segments.  One workgroup; put(at, n, row, b,
-// len) is called by all of its lanes together, n = 0 for lanes without a row.
-template <typename PT, typename F>
-__device__ __forceinline__ void scan_segments(const PT* __restrict__ indptr, int64_t n_rows, int64_t first,
-                                              int64_t seg_len, const build_out& out, int64_t* s_wave,
-                                              int64_t* n_segments, F&& put) {
+// Segment j of the n that a row's [b, b + len) is cut into; `at` is below max_segments.
+__device__ __forceinline__ void write_segment(const build_out& out, int64_t at, int64_t j, int64_t n, int64_t row,
+                                              int64_t b, int64_t len) {
+  out.seg_row[at] = static_cast<int32_t>(row);
+  out.seg_begin[at] = b + len * j / n;
+  out.seg_end[at] = b + len * (j + 1) / n;
+}
+
+// Segments of the long rows rows[first, n_rows): row i of them is cut evenly
+// into ceil(len / seg_len) segments.  Every one of `parts` workgroups scans all
+// rows' counts, 1024 at a time; workgroup `part` writes the rows of every
+// parts-th 1024: a lane by itself those of few segments, a wave together those
+// of more (one lane takes 0.6 us a segment: two divisions and three stores
+// after one another).  Rows of very many are shared between the workgroups.
+constexpr int kLaneSegments = 16;
+constexpr int kWaveSegments = 1024;
+template <typename PT>
+__device__ __forceinline__ void write_segments(const PT* __restrict__ indptr, int64_t n_rows, int64_t first,
+                                               int64_t seg_len, const build_out& out, int64_t* s_wave,
+                                               int64_t* n_segments, int64_t part, int64_t parts) {
   int64_t n_long = n_rows - first;
   if (n_long > out.max_long) n_long = out.max_long;
   int64_t carry = 0;
@@ -135,41 +153,28 @@ __device__ __forceinline__ void scan_segments(const PT* __restrict__ indptr, int
     }
     int64_t total;
     const int64_t at = carry + block_scan(n, s_wave, total) - n;
-    if (live) out.long_seg_ptr[i] = at;
-    put(at, n, row, b, len);
     carry += total;
+    if (live && part == 0) out.long_seg_ptr[i] = at;
+    const bool mine = (base / kBuildThreads) % parts == part;  // uniform
+    const bool few = n <= kLaneSegments;
+    if (mine && few) {
+      for (int64_t j = 0; j < n && at + j < out.max_segments; ++j) write_segment(out, at + j, j, n, row, b, len);
+    }
+    for (uint64_t left = __ballot(!few); left != 0; left &= left - 1) {  // wave-uniform
+      const int from = __ffsll(static_cast<unsigned long long>(left)) - 1;
+      const int64_t n_w = __shfl(n, from);
+      const bool shared = n_w > kWaveSegments;
+      if (!mine && !shared) continue;
+      const int64_t at_w = __shfl(at, from), row_w = __shfl(row, from), b_w = __shfl(b, from), len_w = __shfl(len, from);
+      const int64_t step = shared ? parts * 64 : 64;
+      for (int64_t j = (shared ? part * 64 : 0) + (threadIdx.x & 63); j < n_w && at_w + j < out.max_segments; j += step) {
+        write_segment(out, at_w + j, j, n_w, row_w, b_w, len_w);
+      }
+    }
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && part == 0) {
     if (n_long > 0) out.long_seg_ptr[n_long] = carry;
     *n_segments = carry;
-  }
-}
-
-// Segment j of the n that a row's [b, b + len) is cut into; `at` is below max_segments.
-__device__ __forceinline__ void write_segment(const build_out& out, int64_t at, int64_t j, int64_t n, int64_t row,
-                                              int64_t b, int64_t len) {
-  out.seg_row[at] = static_cast<int32_t>(row);
-  out.seg_begin[at] = b + len * j / n;
-  out.seg_end[at] = b + len * (j + 1) / n;
-}
-
-// One wave writes the segments of its lanes' rows: a lane by itself for a row
-// of few, all lanes together for a row of many (one lane took 0.6 us a segment,
-// two divisions and three stores after one another).
-constexpr int kLaneSegments = 4;
-__device__ __forceinline__ void write_segments(const build_out& out, int64_t at, int64_t n, int64_t row, int64_t b,
-                                               int64_t len) {
-  const bool few = n <= kLaneSegments;
-  if (few) {
-    for (int64_t j = 0; j < n && at + j < out.max_segments; ++j) write_segment(out, at + j, j, n, row, b, len);
-  }
-  for (uint64_t left = __ballot(!few); left != 0; left &= left - 1) {  // wave-uniform
-    const int from = __ffsll(static_cast<unsigned long long>(left)) - 1;
-    const int64_t at_w = __shfl(at, from), n_w = __shfl(n, from), row_w = __shfl(row, from), b_w = __shfl(b, from),
-                  len_w = __shfl(len, from);
-    for (int64_t j = threadIdx.x & 63; j < n_w && at_w + j < out.max_segments; j += 64) {
-      write_segment(out, at_w + j, j, n_w, row_w, b_w, len_w);
-    }
   }
 }
 
@@ -234,10 +239,7 @@ __global__ __launch_bounds__(kBuildThreads) void plan_small_kernel(const PT* __r
     }
     __syncthreads();  // the last one also orders the row ids before their reads below
   }
-  scan_segments(indptr, n_rows, s_off[n_bins - 1], seg_len, out, s_wave, &out.meta[kMetaStats + n_bins + 1],
-                [&](int64_t at, int64_t n, int64_t row, int64_t b, int64_t len) {
-                  write_segments(out, at, n, row, b, len);
-                });
+  write_segments(indptr, n_rows, s_off[n_bins - 1], seg_len, out, s_wave, &out.meta[kMetaStats + n_bins + 1], 0, 1);
 }
 
 // Workgroup b counts the bins of rows [1024 b, 1024 (b + 1)) into
@@ -316,39 +318,11 @@ __global__ __launch_bounds__(kBuildThreads) void plan_reduce_kernel(const PT* __
 }
 
 template <typename PT>
-__global__ __launch_bounds__(kBuildThreads) void plan_ranges_kernel(const PT* __restrict__ indptr, int64_t n_rows,
-                                                                    int n_bins, int64_t seg_len, build_out out) {
+__global__ __launch_bounds__(kBuildThreads) void plan_segments_kernel(const PT* __restrict__ indptr, int64_t n_rows,
+                                                                      int n_bins, int64_t seg_len, build_out out) {
   __shared__ int64_t s_wave[kBuildWaves];
-  scan_segments(indptr, n_rows, out.meta[kMetaStats + n_bins - 1], seg_len, out, s_wave,
-                &out.meta[kMetaStats + n_bins + 1], [](int64_t, int64_t, int64_t, int64_t, int64_t) {});
-}
-
-// The segments themselves, a thread each: thread s finds its row in the ranges.
-template <typename PT>
-__global__ __launch_bounds__(FSP_WG_THREADS) void plan_segments_kernel(const PT* __restrict__ indptr, int64_t n_rows,
-                                                                       int n_bins, build_out out) {
-  const int64_t first = out.meta[kMetaStats + n_bins - 1];
-  int64_t n_long = n_rows - first;
-  if (n_long > out.max_long) n_long = out.max_long;
-  int64_t n_seg = out.meta[kMetaStats + n_bins + 1];
-  if (n_seg > out.max_segments) n_seg = out.max_segments;
-  if (n_long <= 0) return;
-  for (int64_t s = static_cast<int64_t>(blockIdx.x) * FSP_WG_THREADS + threadIdx.x; s < n_seg;
-       s += static_cast<int64_t>(gridDim.x) * FSP_WG_THREADS) {
-    int64_t lo = 0, hi = n_long;  // long_seg_ptr[lo] <= s < long_seg_ptr[hi]
-    while (hi - lo > 1) {
-      const int64_t mid = (lo + hi) >> 1;
-      if (out.long_seg_ptr[mid] <= s) {
-        lo = mid;
-      } else {
-        hi = mid;
-      }
-    }
-    const int64_t at = out.long_seg_ptr[lo], n = out.long_seg_ptr[lo + 1] - at;
-    const int64_t row = out.rows[first + lo];
-    const int64_t b = static_cast<int64_t>(indptr[row]);
-    write_segment(out, s, s - at, n, row, b, static_cast<int64_t>(indptr[row + 1]) - b);
-  }
+  write_segments(indptr, n_rows, out.meta[kMetaStats + n_bins - 1], seg_len, out, s_wave,
+                 &out.meta[kMetaStats + n_bins + 1], blockIdx.x, gridDim.x);
 }
 
 static inline int64_t build_row_blocks(int64_t n_rows) {
@@ -363,9 +337,10 @@ static inline int64_t build_blocks(int64_t n_rows, int64_t nnz) {
   const int64_t r = build_row_blocks(n_rows);
   return c > r ? c : r;
 }
+// Workgroups that write the segments, of which the caller provides for max_segments.
 static inline int64_t segment_blocks(int64_t max_segments) {
-  const int64_t b = ceil_div(max_segments, int64_t(FSP_WG_THREADS));
-  return b < 2048 ? b : 2048;
+  const int64_t b = ceil_div(max_segments, int64_t(1024));
+  return b < 1 ? 1 : (b < 64 ? b : 64);
 }
 
 }  // namespace fsp
@@ -440,11 +415,8 @@ int fsp_csr_build_plan(int32_t indptr_type, const void* indptr_dev, int32_t inde
                          ip, n_rows, n_bins, bb, counts, row_blocks, rows_dev);
       st = check_launch("bins_scatter");
       if (st) return st;
-      hipLaunchKernelGGL(plan_ranges_kernel<PT>, dim3(1), dim3(kBuildThreads), 0, s, ip, n_rows, n_bins, seg_len, out);
-      st = check_launch("plan_ranges");
-      if (st || max_segments == 0) return st;
       hipLaunchKernelGGL(plan_segments_kernel<PT>, dim3(static_cast<unsigned>(segment_blocks(max_segments))),
-                         dim3(FSP_WG_THREADS), 0, s, ip, n_rows, n_bins, out);
+                         dim3(kBuildThreads), 0, s, ip, n_rows, n_bins, seg_len, out);
       return check_launch("plan_segments");
     });
   });

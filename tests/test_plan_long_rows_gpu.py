@@ -23,8 +23,11 @@ def _pointer(n_rows, long_rows, device, pt=torch.int32):
 @pytest.mark.parametrize("n_rows,long_rows", [
     (1, {0: 3_000_001}), (1, {0: 1 << 20}), (300, {7: 120_000}), (300, {7: 4_000_000, 8: 65, 299: 192, 0: 193}),
     (500, {i: 193 + i for i in range(500)}), (8193, {0: 100_000, 8192: 64 * 48 + 1}),
+    (300, {0: 60_000, 5: 1024 * 48 + 1, 9: 1024 * 48, 11: 16 * 48 + 1, 12: 16 * 48, 13: 17 * 48}),
+    (9000, {0: 60_000, 5: 1024 * 48 + 1, 9: 1024 * 48, 11: 16 * 48 + 1, 12: 16 * 48, 13: 17 * 48}),
+    (9000, {i: 2000 + i for i in range(0, 9000, 3)}),
     (70_000, {**{i: 200 + i % 900 for i in range(0, 70_000, 31)}, 69_999: 5_000_000}),
-], ids=["one", "one_wave", "small", "mixed", "all", "rows", "many"])
+], ids=["one", "one_wave", "small", "mixed", "all", "rows", "steps_small", "steps", "mid", "many"])
 def test_segments_of_long_rows(device, pt, n_rows, long_rows):
     lengths, indptr, p = _pointer(n_rows, long_rows, device, pt)
     cfg = _plan.spmm_config(16, long_threshold=64, seg_len=48)
