@@ -721,14 +721,9 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
     // pointers and 64-bit offsets the f64 N = 75 product above took 301 us
     // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.  Groups of one
     // or two lanes are the other way round (104608-node graph, int64 indices,
-    // f32 N = 8: 28.7 us with 64-bit offsets, 29.6 us with 32-bit ones), and so
-    // is the paced loop in f32 (power-law rows, int64 indices, N = 64, 96 MiB of
-    // B: 232.6 / 234.5 us; N = 256, 72 MiB: 270.3 / 279.7), though not in f64
-    // (N = 64, 72 MiB: 256.8 / 255.5) and bf16 (N = 128, 64 MiB: 231).
+    // f32 N = 8: 28.7 us with 64-bit offsets, 29.6 us with 32-bit ones).
     const int64_t lim = int64_t(1) << 32;
-    const bool paced_f32 = std::is_same<TV, float>::value && sizeof(T) == 4 &&
-                           spmm_paced(sizeof(T), g_log2, x.n_dense, x.b_rows * x.ldb * (int64_t)sizeof(T), SDD);
-    const bool off32 = (std::is_same<PT, int32_t>::value || (G >= 4 && !paced_f32)) && (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
+    const bool off32 = (std::is_same<PT, int32_t>::value || G >= 4) && (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
                        x.nnz * (int64_t)sizeof(TV) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
                        x.nnz * (int64_t)sizeof(QT) < lim && x.b_rows * x.ldb * (int64_t)sizeof(T) < lim &&
                        x.n_rows * x.ldc * (int64_t)sizeof(T) < lim && partial_bytes < lim &&
