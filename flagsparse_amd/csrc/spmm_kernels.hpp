@@ -351,9 +351,11 @@ struct buffer {
 
 // Workgroups per CU (waves per SIMD) the registers must allow: the most that
 // spills nothing (eight vectors of 16-bit elements need 95 registers; held to 80
-// they spill, and 200000 nodes, N = 128, unroll 8 took 116 us, 87 without).
-template <int UNROLL, bool SDD, int ELEM>
-constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : 8) : (SDD ? 4 : (ELEM == 2 ? 5 : 6));
+// they spill, and 200000 nodes, N = 128, unroll 8 took 116 us, 87 without; with
+// the values behind a permutation unroll 4 needs 66, and held to 64 a bf16 product of
+// N = 256 took 55 us, 50 without).
+template <int UNROLL, bool SDD, bool PERM, int ELEM>
+constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : (PERM && ELEM == 2 ? 7 : 8)) : (SDD ? 4 : (ELEM == 2 ? 5 : 6));
 
 // The same layout and summation order as spmm_slots_kernel (bitwise equal),
 // with the id and value of a nonzero loaded once per quad (LANES 4) or row of
@@ -375,7 +377,7 @@ constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : 8) : (SDD ? 4 : (ELEM == 2 ?
 // kernel: 84.6 -> 80.7 us, its backward 130.5 -> 127.1 us.
 template <typename T, typename TV, typename IT, typename PT, typename QT, int VEC, int UNROLL, int LANES, bool PERM,
           bool SDD, bool TAIL>
-__global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cast<int>(sizeof(T))>)) void spmm_bins_kernel(
+__global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, PERM, static_cast<int>(sizeof(T))>)) void spmm_bins_kernel(
     const PT* __restrict__ indptr, const IT* __restrict__ indices, const TV* __restrict__ data,
     const T* __restrict__ B, int64_t ldb, uint32_t b_bytes, T* __restrict__ C, int64_t ldc, int64_t n_dense, uint32_t nnz,
     int g_log2, typename acc_of<TV>::type* __restrict__ partials, launch_table tab, sdd_args<T, QT> sd) {
@@ -479,9 +481,15 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = A(0);
     P p = beg + slot;
-    bool more = __ballot(p < end) != 0;  // wave-uniform: every lane takes part in the broadcasts
-    if (!more && has_next) trip(beg_n + slot, end_n, c, a, pq);
-    while (more) {
+    bool prefetched = false;  // wave-uniform
+    // wave-uniform: every lane takes part in the broadcasts.  (`more` says the same
+    // as the ballot of the plain product, which makes the compiler keep a first trip
+    // apart from the others, whose B rows then wait for the ids alone and not for
+    // the values too: 26841 x 89266, f32 N = 57 21.4 -> 20.5 us.  In the backward
+    // the second copy spills: training step on 200000 nodes, bf16 252 us with it,
+    // 243 without.)
+    bool more = __ballot(p < end) != 0;
+    while (SDD ? more : __ballot(p < end) != 0) {
       O off[kRegs];
       A av[kRegs];
 #pragma unroll
@@ -492,7 +500,8 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
         if constexpr (PERM) a[r] = data_b.load(ok ? static_cast<O>(pq[r]) : kAbsent);
       }
       const P pn = p + (static_cast<P>(kTrip) << s_log2);
-      more = __ballot(pn < end) != 0;
+      const bool more_n = __ballot(pn < end) != 0;
+      if constexpr (SDD) more = more_n;
       IT cn[kRegs];
       TV an[kRegs];
       QT pqn[kRegs];
@@ -511,7 +520,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
         // with nothing next, it touches no memory): under a branch the compiler
         // could not count the loads in flight, and the last B row of the batch
         // would wait for the prefetch too.
-        if constexpr (u0 == 0) trip(more ? pn : beg_n + slot, more ? end : end_n, cn, an, pqn);
+        if constexpr (u0 == 0) trip(more_n ? pn : beg_n + slot, more_n ? end : end_n, cn, an, pqn);
         if constexpr (u0 == 0) {
 #pragma unroll
           for (int r = 0; r < kRegs; ++r) av[r] = static_cast<A>(a[r]);
@@ -553,7 +562,9 @@ __global__ __launch_bounds__(FSP_WG_THREADS, (kMinBlocks<UNROLL, SDD, static_cas
         if constexpr (PERM || SDD) pq[r] = pqn[r];
       }
       p = pn;
+      prefetched = true;
     }
+    if (!prefetched && has_next) trip(beg_n + slot, end_n, c, a, pq);
     // Sum the S slots of a row: lanes that differ only in the slot bits.
     for (int j = 0; j < s_log2; ++j) {
 #pragma unroll
