@@ -300,25 +300,27 @@ constexpr uint32_t kAbsent = ~0u;
 // spmm_bins_kernel wins.  Time of the former over the latter, int32 indices,
 // rows of power-law length (mean 24) with uniform columns / graphs with hub
 // columns (mean 14), which the caches keep:
-//                                   24 MiB       40           48           56           64           96
-//   16 lanes  f32  N =  64      0.995/1.064  0.986/1.030  0.987/1.011  0.979/1.016  0.989/1.007  0.989/1.003
-//             bf16 N = 128      1.012/1.096  1.009/1.040  0.992/1.035  0.986/1.040  1.004/1.027  0.991/1.021
-//   32 lanes  f32  N = 128      0.995/1.057  0.990/1.027  0.963/1.007  0.975/1.015  0.983/0.992  0.978/0.984
-//             f64  N =  64      1.014/1.106  0.975/1.050  0.953/1.038  0.960/1.034  0.972/1.020  0.967/1.003
-//   64 lanes  f64  N = 128      1.085/1.249  1.007/1.121  0.994/1.072  0.994/1.044  0.981/1.086  0.976/1.014
-//   38 of 64  f64  N =  75      1.072/1.324  1.058/1.201  1.066/1.160  1.033/1.128  1.047/1.135  1.017/1.099
-// The limits lie where what one pattern gains is what the other loses: 48 MiB
-// for rows that fill a group of 32 lanes or more (seven lanes in eight), 56 MiB
-// for other groups of 16 or 32.  A 64-lane group with idle lanes is not paced
-// (38 of 64 up to 400 MiB: 1.01-1.14), nor are groups of 8 lanes (f32 N = 32, 32
-// to 128 MiB: 1.00-1.02, f64 N = 16 0.99-1.08) and the backward (32 to 256 MiB:
-// f32 N = 64 1.01-1.12, bf16 N = 128 1.01-1.08, f64 N = 64 1.09-1.27).
+//                                   24 MiB       32           40           48           56           64
+//   16 lanes  f32  N =  64      0.995/1.064  0.997/1.035  0.986/1.030  0.987/1.011  0.979/1.016  0.989/1.007
+//             bf16 N = 128      1.012/1.096  0.991/1.064  1.009/1.040  0.992/1.035  0.986/1.040  1.004/1.027
+//   32 lanes  f32  N = 128      0.995/1.057  0.991/1.037  0.990/1.027  0.963/1.007  0.975/1.015  0.983/0.992
+//             f64  N =  64      1.014/1.106  0.989/1.106  0.975/1.050  0.953/1.038  0.960/1.034  0.972/1.020
+//   64 lanes  f64  N = 128      1.085/1.249  1.036/1.160  1.007/1.121  0.994/1.072  0.994/1.044  0.981/1.086
+//   38 of 64  f64  N =  75      1.072/1.324  1.078/1.252  1.058/1.201  1.066/1.160  1.033/1.128  1.047/1.135
+// Uniform columns gain from the eight L2s' 32 MiB on, graphs from twice that.
+// The limit of rows that fill a group of 32 lanes (seven lanes in eight) is where
+// the former begin to gain, which is the most there is to gain, 5 %; that of other
+// groups of 16 or 32 and of full ones of 64 lies between, where one gains what the
+// other loses.  A 64-lane group with idle lanes is not paced (38 of 64 up to 400
+// MiB: 1.01-1.14), nor are groups of 8 lanes (f32 N = 32, 32 to 128 MiB: 1.00-1.02,
+// f64 N = 16 0.99-1.08) and the backward (32 to 256 MiB: f32 N = 64 1.01-1.12, bf16
+// N = 128 1.01-1.08, f64 N = 64 1.09-1.27).
 constexpr int64_t kPacedBytes = int64_t(56) << 20;
-constexpr int64_t kPacedFullBytes = int64_t(48) << 20;
+constexpr int64_t kPacedFullBytes = int64_t(32) << 20;
 static inline bool spmm_paced(int64_t elem_bytes, int g_log2, int64_t n_dense, int64_t b_bytes, bool backward) {
   const bool full = n_dense * elem_bytes * 8 >= int64_t(16 * 7) << g_log2;
   if (backward || g_log2 < 4 || (g_log2 == 6 && !full)) return false;
-  return b_bytes >= (g_log2 >= 5 && full ? kPacedFullBytes : kPacedBytes);
+  return b_bytes >= (g_log2 == 5 && full ? kPacedFullBytes : kPacedBytes);
 }
 
 // Whether a launch of whole vectors with 32-bit offsets shares its nonzeros

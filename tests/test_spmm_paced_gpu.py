@@ -1,6 +1,6 @@
 """The SpMM's two loops are bitwise equal: the same product with a dense operand
-just below and just at the sizes where the rule changes loops (48 MiB for rows
-that fill a group of 32 lanes or more, 56 MiB for other groups of 16 or 32)."""
+just below and just at the sizes where the rule changes loops (32 MiB for rows
+that fill a group of 32 lanes, 56 MiB for groups of 16, 32 and full ones of 64)."""
 
 import pytest
 import torch
@@ -19,8 +19,8 @@ def _shares(dtype, n, rows):
 
 
 @pytest.mark.parametrize("index", [torch.int32, torch.int64], ids=["i32", "i64"])
-@pytest.mark.parametrize("dtype,n,limit", [(torch.float32, 40, 56), (torch.float32, 64, 56), (torch.float32, 128, 48),
-                                           (torch.float32, 256, 48), (torch.float64, 32, 56), (torch.float64, 64, 48),
+@pytest.mark.parametrize("dtype,n,limit", [(torch.float32, 40, 56), (torch.float32, 64, 56), (torch.float32, 128, 32),
+                                           (torch.float32, 256, 56), (torch.float64, 32, 56), (torch.float64, 64, 32),
                                            (torch.bfloat16, 128, 56), (torch.float16, 200, 56)])
 def test_loops_agree(device, dtype, n, limit, index):
     row_bytes = n * torch.empty(0, dtype=dtype).element_size()
