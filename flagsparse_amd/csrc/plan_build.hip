@@ -126,16 +126,16 @@ __device__ __forceinline__ void write_segment(const build_out& out, int64_t at, 
 
 // Segments of the long rows rows[first, n_rows): row i of them is cut evenly
 // into ceil(len / seg_len) segments.  Every one of `parts` workgroups scans all
-// rows' counts, 1024 at a time; workgroup `part` writes the rows of every
-// parts-th 1024: a lane by itself those of few segments, a wave together those
-// of more (one lane takes 0.6 us a segment: two divisions and three stores
-// after one another).  Rows of very many are shared between the workgroups.
+// rows' counts, 1024 at a time, and writes each parts-th row (a power of two):
+// a lane by itself those of few segments, a wave together those of more (one
+// lane takes 0.6 us a segment: two divisions and three stores after one
+// another).  Rows of very many are shared between the workgroups.
 constexpr int kLaneSegments = 16;
 constexpr int kWaveSegments = 1024;
 template <typename PT>
 __device__ __forceinline__ void write_segments(const PT* __restrict__ indptr, int64_t n_rows, int64_t first,
                                                int64_t seg_len, const build_out& out, int64_t* s_wave,
-                                               int64_t* n_segments, int64_t part, int64_t parts) {
+                                               int64_t* n_segments, unsigned part, unsigned parts) {
   int64_t n_long = n_rows - first;
   if (n_long > out.max_long) n_long = out.max_long;
   int64_t carry = 0;
@@ -155,19 +155,18 @@ __device__ __forceinline__ void write_segments(const PT* __restrict__ indptr, in
     const int64_t at = carry + block_scan(n, s_wave, total) - n;
     carry += total;
     if (live && part == 0) out.long_seg_ptr[i] = at;
-    const bool mine = (base / kBuildThreads) % parts == part;  // uniform
+    const bool mine = (threadIdx.x & (parts - 1)) == part;
     const bool few = n <= kLaneSegments;
     if (mine && few) {
       for (int64_t j = 0; j < n && at + j < out.max_segments; ++j) write_segment(out, at + j, j, n, row, b, len);
     }
-    for (uint64_t left = __ballot(!few); left != 0; left &= left - 1) {  // wave-uniform
+    for (uint64_t left = __ballot(!few && (mine || n > kWaveSegments)); left != 0; left &= left - 1) {  // wave-uniform
       const int from = __ffsll(static_cast<unsigned long long>(left)) - 1;
       const int64_t n_w = __shfl(n, from);
       const bool shared = n_w > kWaveSegments;
-      if (!mine && !shared) continue;
       const int64_t at_w = __shfl(at, from), row_w = __shfl(row, from), b_w = __shfl(b, from), len_w = __shfl(len, from);
-      const int64_t step = shared ? parts * 64 : 64;
-      for (int64_t j = (shared ? part * 64 : 0) + (threadIdx.x & 63); j < n_w && at_w + j < out.max_segments; j += step) {
+      const int64_t step = shared ? int64_t(parts) * 64 : 64;
+      for (int64_t j = (shared ? int64_t(part) * 64 : 0) + (threadIdx.x & 63); j < n_w && at_w + j < out.max_segments; j += step) {
         write_segment(out, at_w + j, j, n_w, row_w, b_w, len_w);
       }
     }
@@ -337,10 +336,12 @@ static inline int64_t build_blocks(int64_t n_rows, int64_t nnz) {
   const int64_t r = build_row_blocks(n_rows);
   return c > r ? c : r;
 }
-// Workgroups that write the segments, of which the caller provides for max_segments.
+// Workgroups that write the segments, of which the caller provides for
+// max_segments: a power of two, one per 1024 up to 64.
 static inline int64_t segment_blocks(int64_t max_segments) {
-  const int64_t b = ceil_div(max_segments, int64_t(1024));
-  return b < 1 ? 1 : (b < 64 ? b : 64);
+  int64_t b = 1;
+  while (b < 64 && b * 1024 < max_segments) b *= 2;
+  return b;
 }
 
 }  // namespace fsp
