@@ -93,6 +93,13 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
   using A = typename acc_of<TV>::type;
   using O = typename addr<OFF32>::off_t;  // element / byte offsets
   using P = typename std::conditional<OFF32, int32_t, int64_t>::type;  // nonzero positions
+  // A column id.  B's offsets fit 32 bits, and so do its rows' numbers: of an
+  // int64 id the low half is loaded.  Loading both, the compiler gave the unused
+  // half's register to the next load's address and waited for every load in
+  // flight between the two (10000 x 86679, power-law rows, f32 N = 128, int64
+  // indices: 40 us, 30 with int32 indices or 64-bit offsets).
+  using I = typename std::conditional<OFF32, uint32_t, IT>::type;
+  constexpr int kIdStride = sizeof(IT) / sizeof(I);
   const int k = find_bin(tab, blockIdx.x);
   const launch_bin lb = tab.b[k];  // a copy: the fields stay in registers
   const int s_log2 = lb.lanes_log2;
@@ -157,13 +164,13 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
   // stay raw: masking or converting them here would make the compiler wait
   // for every load in flight (the B rows included) right after the prefetch,
   // so the mask and the conversion are applied where they are consumed.
-  auto trip = [&](P p, P end, IT (&c)[UNROLL], TV (&a)[UNROLL], QT (&pq)[UNROLL]) {
+  auto trip = [&](P p, P end, I (&c)[UNROLL], TV (&a)[UNROLL], QT (&pq)[UNROLL]) {
     const P last = end > 0 ? end - 1 : P(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       const P q = p + static_cast<P>(u) * S;
       const O qc = static_cast<O>(q < end ? q : last);
-      c[u] = elem<OFF32>(indices, qc);
+      c[u] = elem<OFF32>(reinterpret_cast<const I*>(indices), qc * static_cast<O>(kIdStride));
       const O qv = PERM ? static_cast<O>(elem<OFF32>(perm, qc)) : qc;
       a[u] = elem<OFF32>(data, qv);
       if constexpr (SDD) pq[u] = elem<OFF32>(sd.pos, qc);
@@ -183,7 +190,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
   O out, jrow;
   P beg, end;
   item(rr, out, beg, end, jrow);
-  IT c[UNROLL];
+  I c[UNROLL];
   TV a[UNROLL];
   QT pq[UNROLL];
   trip(beg + slot, end, c, a, pq);
@@ -214,7 +221,7 @@ __global__ __launch_bounds__(FSP_WG_THREADS) void spmm_slots_kernel(
       const bool same = pn < end;
       prefetched = prefetched || !same;
       TV an[UNROLL];
-      IT cn[UNROLL];
+      I cn[UNROLL];
       QT pqn[UNROLL];
       if constexpr (SDD) {
         // unconditional (with nothing next it reloads this trip's nonzeros,
