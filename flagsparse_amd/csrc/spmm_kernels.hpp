@@ -379,7 +379,7 @@ constexpr int kMinBlocks = UNROLL <= 4 ? (SDD ? 5 : (PERM && ELEM == 2 ? 7 : 8))
 // that no lane needs are skipped.  That takes both zeros: the next rows'
 // nonzeros are loaded in the wave's last trip and no sooner, or an infinite
 // value among them would meet the zeros of a row that has ended.  Against
-// spmm_slots_kernel, vector instructions per launch fall from 44.6 to 23.7
+// spmm_slots_kernel, vector instructions per launch fall from 44.6 to 23.8
 // million and loads from 6.0 to 2.6 million (262144 x 229376, f32 N = 64, either
 // side of the limit above).  100003 x 70001 f64, N = 75: 290 -> 240 us;
 // 1024-matrix batch, N = 32: 687 -> 665 us; 200000-node graph, bf16 N = 128, by
@@ -740,8 +740,9 @@ static int launch_spmm(const spmm_args& x, const fsp_csr_plan* plan, hipStream_t
     // whatever the row pointer's type (its values fit then too).  With 64-bit
     // pointers and 64-bit offsets the f64 N = 75 product above took 301 us
     // against 290 us, the K = 128 f32 SDDMM 192 against 189 us.  Groups of one
-    // or two lanes are the other way round (104608-node graph, int64 indices,
-    // f32 N = 8: 28.7 us with 64-bit offsets, 29.6 us with 32-bit ones).
+    // or two lanes are the other way round or even (int64 indices, 64-bit offsets
+    // / 32-bit ones: 104608-node graph, bf16 N = 16 20.7 / 21.4 us, f32 N = 8 21.2
+    // / 21.2; 150000 uniform rows, f64 N = 4 34.1 / 35.4).
     const int64_t lim = int64_t(1) << 32;
     const bool off32 = (std::is_same<PT, int32_t>::value || G >= 4) && (!(PERM || SDD) || std::is_same<QT, int32_t>::value) &&
                        x.nnz * (int64_t)sizeof(TV) < lim && x.nnz * (int64_t)sizeof(IT) < lim &&
